@@ -84,6 +84,7 @@ struct Step {
     std::vector<unsigned char> arg;   // kernel argument block (a POD struct)
     int in_field = 0, out_field = 0;  // byte offsets of the in/out pointers in arg
     int nt_field = -1;                // byte offset of KArgs::nt in arg, if any
+    int nt_mask = 3;                  // NT_STORE / NT_LOAD flags that may be set there
     std::string name;
 };
 

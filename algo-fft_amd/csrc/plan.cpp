@@ -16,7 +16,7 @@
 #include <cmath>
 
 #include "afft_internal.hpp"
-#include "kgen.hpp"
+#include "kmix.hpp"
 
 namespace afft {
 
@@ -432,9 +432,7 @@ static int emit_fourstep(Plan& p, int di, const AxisJob& j, std::string& algo) {
 }
 
 // ---- runtime-size mixed radix ------------------------------------------------
-const void* gen_kernel(int prec, int var, int dir);
-const void* gen_ip_kernel(int prec, int dir);
-const void* gen_ipg_kernel(int prec, int var, int dir);
+const void* mix_kernel(int prec, int var, int dir);
 const void* copy_kernel(int prec);
 
 // Radix schedule for a 2/3/5/7-smooth n: radix-16 passes and the
@@ -471,87 +469,10 @@ std::vector<int> smooth_schedule(int64_t n) {
 int gen_cap(int prec) { return prec ? 4096 : 8192; }
 int gen_row_cap(int prec) { return prec ? 8192 : 16384; }
 
-// Threads resident per CU for blocks of `threads` threads and `lds` bytes
-// of LDS, at `wps` waves per SIMD (the kernel's register use): blocks
-// counted by LDS (160 KiB) and by wave slots.
-static int64_t gen_resident(int threads, int64_t lds, int wps) {
-    const int64_t lds_blocks = std::max<int64_t>(1, (int64_t)(160 << 10) / std::max<int64_t>(1, lds));
-    const int64_t wave_blocks = std::max(1, wps / ((threads / 64 + 3) / 4));
-    return std::min(lds_blocks, wave_blocks) * threads;
-}
-
-// Threads of an in-place row block: the multiple of 64 from n/16 (each pass
-// holds at most 16 points of a thread) up to the kernel's maximum that keeps
-// the most threads resident per CU; on a tie the smaller block.  E.g.
-// complex64 N=8000 (64 KiB): 512 threads, two blocks (0.334 ms) against 704
-// threads, one block (0.481 ms).
-static int gen_ip_threads(int64_t n, int prec, int64_t* resident = nullptr) {
-    const int64_t es = prec ? 16 : 8;
-    const int maxt = prec ? GenIP<double>::THREADS : GenIP<float>::THREADS;
-    const int wps = prec ? GenIP<double>::WAVES_PER_SIMD : GenIP<float>::WAVES_PER_SIMD;
-    int best = maxt;
-    int64_t best_res = -1;
-    for (int tt = (int)(((n + 15) / 16 + 63) / 64 * 64); tt <= maxt; tt += 64) {
-        const int64_t res = gen_resident(tt, n * es, wps);
-        if (res > best_res) { best_res = res; best = tt; }
-    }
-    if (resident) *resident = best_res;
-    return best;
-}
-
 int64_t next_pow2(int64_t n) {
     int64_t m = 1;
     while (m < n) m <<= 1;
     return m;
-}
-
-struct GenCfg {
-    int tpt, g, threads;
-    int lds;
-    bool ipg = false;   // k_gen_ipg: G transforms per block, passes in place in one buffer
-};
-
-// Two LDS buffers of G transforms, TPT threads each.  Row layouts: about 8
-// points per thread up to 256 threads, and one transform per block above
-// 4096 points: 1024 threads for complex64 (the LDS of two buffers allows one
-// block per CU, so its waves are all the latency hiding there is), 512 for
-// complex128.  Column layouts keep about 16 points per thread: more adjacent
-// columns per block make longer coalesced segments.  Measured on 512 MiB
-// batches: N=1000 rows 0.37 -> 0.26 ms, N=6000 rows 0.65 -> 0.50 ms (512
-// threads) -> 0.45 ms (1024 threads); column passes lose with fewer columns
-// per block.
-static GenCfg gen_cfg_2b(int64_t n, int prec, bool rows) {
-    GenCfg c;
-    if (rows && n > 4096) c.tpt = prec == 0 ? GEN_ROWTHREADS : GEN_MAXTHREADS;
-    else if (rows) c.tpt = (int)std::min<int64_t>(GEN_THREADS, next_pow2((n + 7) / 8));
-    else c.tpt = (int)std::min<int64_t>(GEN_THREADS, next_pow2((n + 15) / 16));
-    c.threads = std::max(GEN_THREADS, c.tpt);
-    c.g = c.threads / c.tpt;
-    c.lds = (int)(2 * c.g * n * (prec ? 16 : 8));
-    return c;
-}
-
-// Contiguous rows run one transform per block with every pass in place in
-// one LDS buffer (k_gen_ip) above the two-buffer kernel's reach (8192
-// complex64 / 4096 complex128 points), and below it where that keeps at
-// least twice the threads resident per CU of the two-buffer layout, whose
-// rows hold 2n points (k_gen rows take 94-97 VGPRs for complex64, 4 waves
-// per SIMD, and 165 for complex128, 3), or as many where the two-buffer
-// layout runs a single block per CU.  Measured on 512 MiB batches
-// (two-buffer -> in place): complex64 N=3500 0.416 -> 0.313 ms, N=4000
-// 0.409 -> 0.323 ms (two blocks of 256 threads against four), N=4500 0.445
-// -> 0.417 ms (one block of 1024 threads against two of 512), N=6000 0.387
-// -> 0.365 ms, N=8000 0.349 -> 0.334 ms; complex128 N=3000 0.489 -> 0.328
-// ms.  Kept on the two-buffer kernel: complex64 N=3000 (three blocks of 256
-// against four: 0.341 against 0.350 ms), N=2000 (0.265 against 0.396 ms),
-// complex128 N=2500 (0.290 against 0.335 ms).
-static bool gen_use_ip(int64_t n, int prec) {
-    if (n > gen_cap(prec)) return true;
-    const GenCfg c = gen_cfg_2b(n, prec, true);
-    int64_t res_ip = 0;
-    gen_ip_threads(n, prec, &res_ip);
-    const int64_t res_2b = gen_resident(c.threads, c.lds, prec ? 3 : 4);
-    return res_ip >= 2 * res_2b || (res_ip >= res_2b && res_2b == c.threads);
 }
 
 // Whether one runtime-radix launch holds a transform of n points on this
@@ -560,105 +481,250 @@ static bool gen_single_fits(int prec, int64_t n, bool rows) {
     return n <= gen_cap(prec) || (rows && n <= gen_row_cap(prec));
 }
 
-// With ipg, column layouts (both four-step passes, strided axes of N-D
-// plans) run in place in one LDS buffer (k_gen_ipg) when they hold at most
-// 16 points per thread: half the LDS of the two-buffer kernel, so twice the
-// blocks per CU.  Measured on 512 MiB batches: complex64 N=100000 (250 x
-// 400) 0.990 -> 0.831 ms, N=250000 (500 x 500) 1.012 -> 0.829 ms,
-// complex128 N=100000 0.952 -> 0.700 ms.  Strided axes gain once blocks
-// grow to 512 threads (below): complex64 1200 x 1500 1.325 -> 0.812 ms,
-// 1000 x 1000 0.791 -> 0.570 ms, 250 x 250 x 64 1.179 -> 0.860 ms;
-// complex128 1200 x 1500 0.752 -> 0.656 ms, 1000 x 1000 0.755 -> 0.618 ms
-// (at 256 threads the in-place form had lost 2-7 % on them).
-static GenCfg gen_cfg(int64_t n, int prec, bool rows, bool ipg = false) {
-    if (rows && gen_use_ip(n, prec)) {
-        GenCfg c;
-        c.tpt = c.threads = gen_ip_threads(n, prec);
-        c.g = 1;
-        c.lds = (int)(n * (prec ? 16 : 8));
-        return c;
+// Shape of one k_mix launch.
+struct MixShape {
+    std::vector<int> rad;
+    int tpt = 1, g = 1, threads = 64, lds = 0, pitch = 0;
+};
+enum MixLayout { MIX_ROWS = 0, MIX_COLS = 1, MIX_TROWS = 2 };   // VAR_ROW; VAR_COL and VAR_4A; VAR_4B
+
+// Mean number of LDS bank passes beyond the first of a wave's access to the
+// points addr(lane) (< 0: idle lane): the 64 banks of 4 bytes serve 256 bytes
+// at a time, 32 complex64 or 16 complex128 points.
+template <class Addr>
+static double bank_excess(int per, Addr addr) {
+    int sum = 0, groups = 0;
+    for (int h = 0; h < 64; h += per) {
+        int cnt[32] = {0}, mx = 0;
+        for (int l = h; l < h + per; ++l) {
+            const int64_t x = addr(l);
+            if (x >= 0) mx = std::max(mx, ++cnt[x % per]);
+        }
+        if (mx) { sum += mx; ++groups; }
     }
-    GenCfg c = gen_cfg_2b(n, prec, rows);
-    if (ipg && !rows && n <= 16 * (int64_t)c.tpt) {
-        c.ipg = true;
-        // Blocks of 512 threads where 256 would hold fewer than 16
-        // (complex64) / 4 (complex128) transforms: longer column segments.
-        // Measured on 512 MiB batches (256 -> 512 threads), complex64:
-        // N=36000 (32 x 1125) 1.45 -> 0.85 ms, N=10^6 (1000 x 1000) 1.22 ->
-        // 0.72 ms, N=100000 0.82 -> 0.71 ms, but N=24000 (64 x 375) 0.60 ->
-        // 0.62 ms and N=162000 (400 x 405) 0.83 -> 0.88 ms; complex128
-        // N=36000 0.84 -> 0.69 ms, while N=10^6 (4 transforms a block at 256)
-        // went 0.71 -> 0.78 ms and N=100000 0.70 -> 0.77 ms.
-        if (c.g < (prec ? 4 : 16))
-            c.threads = std::min(2 * c.threads, prec ? GenIPG<double>::THREADS : GenIPG<float>::THREADS);
-        c.g = c.threads / c.tpt;
-        c.lds = (int)(c.g * n * (prec ? 16 : 8));
-    }
-    return c;
+    return groups ? (double)sum / groups - 1.0 : 0.0;
 }
 
-// ipg: may choose the in-place grouped kernel (four-step passes); *ipg says
-// whether it did, and lds is then that kernel's.
-static int gen_args(Plan& p, int64_t n, bool rows, GArgs& g, int* tpt, int* lds, int* threads,
-                    bool* ipg = nullptr) {
-    std::vector<int> rad = smooth_schedule(n);
-    if (rad.empty() || (int)rad.size() > GEN_MAXPASS) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule");
-    KernelInfo fake{};
-    fake.prec = p.desc.precision;
-    // reuse the schedule twiddle generator with the runtime radix list
+static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout lay) {
+    const int per = prec ? 16 : 32;
+    double out = 0;
+    int64_t ns = 1;
+    for (size_t i = 0; i < m.rad.size(); ++i) {
+        const int64_t q = m.rad[i], nr = n / q;
+        const bool lanes_c = lay == MIX_COLS || (lay == MIX_TROWS && i + 1 == m.rad.size());
+        auto at = [&](int l, bool write) -> int64_t {
+            const int64_t c = lanes_c ? l % m.g : l / m.tpt, j = lanes_c ? l / m.g : l % m.tpt;
+            if (l >= m.g * m.tpt || j >= nr) return -1;
+            const int64_t k = j % ns, x = write ? (j - k) * q + k : j;
+            return lay == MIX_COLS ? x * m.g + c : c * m.pitch + x;
+        };
+        if (i) out += bank_excess(per, [&](int l) { return at(l, false); });
+        if (i + 1 < m.rad.size()) out += bank_excess(per, [&](int l) { return at(l, true); });
+        ns *= q;
+    }
+    return out;
+}
+
+// Estimated cost of a launch shape, in passes, without the bank conflicts:
+// the passes, the lane slots beyond one per point and pass, the resident
+// blocks per CU (LDS, and 5 / 3 waves per SIMD), whether there is only one,
+// the line segments of the global accesses and the block size.  The
+// coefficients are fitted on all schedules, thread counts and group sizes
+// of 70 row lengths (24 .. 16128 points), 52 column and 26 transposing cases
+// of 512 MiB in both precisions: the pick is on average 2.4 % (rows), 4.4 %
+// (columns) and 6.6 % (transposing rows) slower than the best one, 25 % at
+// worst.
+static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total) {
+    const int es = prec ? 16 : 8, wps = prec ? 3 : 5, waves = m.threads / 64;
+    const int by_waves = waves <= 8 ? wps * 4 / waves : wps / ((waves + 3) / 4);
+    const int blocks = std::max(1, std::min({(int)(163840 / std::max(m.lds, 1)), by_waves, 32}));
+    const double P = (double)m.rad.size(), inv = 1.0 / blocks, one = blocks == 1 ? 1.0 : 0.0, th = m.threads / 1024.0;
+    double work = -P;
+    for (int q : m.rad) {
+        const int64_t nr = n / q;
+        work += (double)m.threads / m.g * ((nr + m.tpt - 1) / m.tpt) * q / n;
+    }
+    const double seg = m.g * es, seg128 = std::max(0.0, 128 / seg - 1), seg64 = seg < 64 ? 1.0 : 0.0;
+    const double rl = 128.0 / (std::min<int64_t>(m.tpt, n / m.rad.front()) * es);
+    const double rs = 128.0 / (std::min<int64_t>(m.tpt, n / m.rad.back()) * es);
+    // fewer blocks than CUs: smaller groups spread the work
+    const double idle = blocks_total < 256 ? std::log2(256.0 / blocks_total) : 0.0;
+    switch (lay) {
+    case MIX_ROWS:
+        return P + 0.105 * work + 0.538 * inv + 0.113 * one + 0.056 * rl + 0.035 * rs + 0.029 * rl * rl +
+               0.037 * rs * rs - 0.433 * th + idle;
+    case MIX_COLS:
+        return P + 0.546 * work + 1.647 * inv + 3.575 * one + 1.155 * seg128 + 1.173 * seg64 - 1.645 * th + idle;
+    default:
+        return P + 0.054 * work + 1.81 * inv + 0.05 * one + 0.886 * seg128 + 0.106 * seg64 + 0.205 * rl -
+               0.0092 * m.rad.front() - 0.143 * th + idle;
+    }
+}
+
+static constexpr int kMixRadices[] = {20, 18, 16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+
+// Fewest passes of a 7-smooth n over kMixRadices (at most `most`).
+static int mix_min_passes(int64_t n, int most) {
+    if (n == 1) return 0;
+    if (most <= 0) return MIX_MAXPASS + 1;
+    int best = MIX_MAXPASS + 1;
+    for (int q : kMixRadices)
+        if (n % q == 0) best = std::min(best, 1 + mix_min_passes(n / q, std::min(most, best - 1) - 1));
+    return best;
+}
+
+// Launch shape of n 7-smooth points: every order of radices with the fewest
+// passes, and with one more where they are within a factor 1.7 of each
+// other, times every thread count that gives some pass whole butterflies,
+// times the group sizes; the bank conflicts rank the cheapest of them.
+// Radices up to 10 hold 16 points per thread, so at most n/16 threads (the
+// largest block at the largest length) always fit.
+static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out) {
+    const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
+    const double conf = lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012;
+    const int minp = mix_min_passes(n, MIX_MAXPASS);
+    if (minp > MIX_MAXPASS) return false;
+    std::vector<std::pair<double, MixShape>> top;   // sorted, the cheapest few
+    constexpr size_t KEEP = 12;
+    std::vector<int> rad;
+    auto consider = [&]() {
+        int lo = 1;
+        for (int q : rad) lo = std::max<int>(lo, (int)((n / q + mix_mb(q) - 1) / mix_mb(q)));
+        int tpts[64], nt = 0;
+        for (int q : rad)
+            for (int m = 1; m <= mix_mb(q); ++m) {
+                const int64_t t = (n / q + m - 1) / m;
+                if (t < lo || t > maxth) continue;
+                bool seen = false;
+                for (int i = 0; i < nt; ++i) seen |= tpts[i] == t;
+                if (!seen && nt < 64) tpts[nt++] = (int)t;
+            }
+        for (int i = 0; i < nt; ++i) {
+            MixShape m;
+            m.tpt = tpts[i];
+            int last_g = 0;
+            for (int w = 0; w < 6; ++w) {
+                if (lay == MIX_ROWS) {
+                    static constexpr int want[6] = {64, 128, 192, 256, 512, 0};
+                    if (!want[w]) break;
+                    m.g = (int)std::min<int64_t>(count, std::max(1, want[w] / m.tpt));
+                } else {
+                    m.g = 32 >> w;
+                }
+                if (m.g == last_g) continue;
+                last_g = m.g;
+                if (m.g > 1 && m.g >= 2 * count) continue;
+                m.pitch = (int)(lay == MIX_TROWS ? n | 1 : n);
+                const int64_t lds = (int64_t)m.g * m.pitch * es;
+                if ((int64_t)m.g * m.tpt > maxth || lds > 163840) continue;
+                m.lds = (int)lds;
+                m.threads = (m.g * m.tpt + 63) / 64 * 64;
+                m.rad = rad;
+                const double c = mix_cost(m, n, prec, lay, std::max<int64_t>(1, (count + m.g - 1) / m.g * slices));
+                if (top.size() == KEEP && c >= top.back().first) continue;
+                auto it = top.begin();
+                while (it != top.end() && it->first <= c) ++it;
+                top.insert(it, {c, m});
+                if (top.size() > KEEP) top.pop_back();
+            }
+        }
+    };
+    auto extend = [&](auto&& self, int64_t rest, int passes) -> void {
+        if (rest == 1) {
+            if ((int)rad.size() != passes) return;
+            if (passes == minp + 1 && !top.empty()) {
+                const auto mm = std::minmax_element(rad.begin(), rad.end());
+                if (*mm.second * 10 > *mm.first * 17) return;
+            }
+            consider();
+            return;
+        }
+        if ((int)rad.size() == passes) return;
+        for (int q : kMixRadices) {
+            if (rest % q) continue;
+            rad.push_back(q);
+            self(self, rest / q, passes);
+            rad.pop_back();
+        }
+    };
+    // more passes only where no schedule of the fewest fits the block size
+    for (int passes = minp; passes <= MIX_MAXPASS && (passes <= minp + 1 || top.empty()); ++passes)
+        extend(extend, n, passes);
+    if (top.empty()) return false;
+    double best = 1e300;
+    for (auto& t : top) {
+        const double c = t.first + conf * mix_bank_excess(t.second, n, prec, lay);
+        if (c < best) {
+            best = c;
+            out = t.second;
+        }
+    }
+    return true;
+}
+
+// Kernel arguments of a launch shape; builds the twiddle tables (the
+// powers mix_twpow of every butterfly, see mix_twiddle).
+static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t slices, MixArgs& a, MixShape& m) {
+    if (smooth_schedule(n).empty() || !mix_shape(n, p.desc.precision, lay, count, slices, m))
+        return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule");
+    a.n = (int)n;
+    a.npass = (int)m.rad.size();
     std::vector<double> tw;
-    int64_t ns = rad[0];
-    g.npass = (int)rad.size();
-    g.ns[0] = 1;
-    g.nsm[0] = mod_magic(1);
-    g.twoff[0] = 0;
-    g.rad[0] = rad[0];
-    for (size_t i = 1; i < rad.size(); ++i) {
-        const int R = rad[i];
-        g.rad[i] = R;
-        g.ns[i] = (int)ns;
-        g.nsm[i] = mod_magic((unsigned)ns);
-        g.twoff[i] = (int)(tw.size() / 2);
-        // k-major (entry k*(R-1) + r-1): the runtime passes read a butterfly's
-        // R-1 twiddles at compile-time offsets from one address
-        for (int64_t kk = 0; kk < ns; ++kk)
-            for (int r = 1; r < R; ++r) {
+    int64_t ns = 1;
+    for (int i = 0; i < a.npass; ++i) {
+        const int R = m.rad[i];
+        a.p[i] = MixPass{R, (int)ns, (int)(n / R), mod_magic((unsigned)ns), (int)(tw.size() / 2)};
+        for (int w = 0; i && w < mix_ntw(R); ++w)
+            for (int64_t k = 0; k < ns; ++k) {
                 double re, im;
-                root_of_unity(kk * r, ns * R, &re, &im);
+                root_of_unity(k * mix_twpow(R, w), ns * R, &re, &im);
                 tw.push_back(re);
                 tw.push_back(im);
             }
         ns *= R;
     }
-    int rc;
+    a.tpt = m.tpt;
+    a.g = m.g;
+    a.divm = mod_magic((unsigned)(lay == MIX_COLS ? m.g : m.tpt));
+    a.pitch = m.pitch;
     if (p.desc.precision == 0) {
         std::vector<float> f(tw.begin(), tw.end());
-        rc = upload_table(p, f.data(), f.size() * 4, &g.k.tw);
-    } else {
-        rc = upload_table(p, tw.data(), tw.size() * 8, &g.k.tw);
+        return upload_table(p, f.data(), f.size() * 4, &a.k.tw);
     }
-    if (rc) return rc;
-    GenCfg c = gen_cfg(n, p.desc.precision, rows, ipg != nullptr);
-    g.n = (int)n;
-    g.tpt = c.tpt;
-    *tpt = c.tpt;
-    *lds = c.lds;
-    *threads = c.threads;
-    if (ipg) *ipg = c.ipg;
-    return AFFT_OK;
+    return upload_table(p, tw.data(), tw.size() * 8, &a.k.tw);
 }
 
-static Step make_gen_step(const void* fn, const GArgs& g, int64_t gx, int lds, int threads, const std::string& name) {
+// Non-temporal accesses pay only where a wave covers whole lines: rows whose
+// first and last passes run at least 512 contiguous bytes (complex64 60
+// points 0.259 -> 0.200 ms without them, 525 0.224 -> 0.204; 960 0.183 ->
+// 0.175 with them), columns whose groups start and end on 128-byte lines
+// (transposing 400-point rows into rows of 500 0.357 -> 0.251 ms without
+// them, into rows of 512 0.196 -> 0.189 with them).
+static int mix_nt_mask(const MixShape& m, const MixArgs& a, MixLayout lay, int prec) {
+    const int es = prec ? 16 : 8;
+    if (lay == MIX_ROWS) {
+        const int run = std::min({m.tpt, a.p[0].nr, a.p[a.npass - 1].nr}) * es;
+        return run >= 512 ? NT_STORE | NT_LOAD : 0;
+    }
+    auto lines = [&](long long nd, long long bd) { return (nd * es) % 128 == 0 && (bd * es) % 128 == 0 && (m.g * es) % 128 == 0; };
+    int nt = lines(a.k.out_nd, a.k.out_bd) ? NT_STORE : 0;
+    if (lay == MIX_COLS && lines(a.k.in_nd, a.k.in_bd)) nt |= NT_LOAD;
+    return nt;
+}
+
+static Step make_mix_step(const void* fn, const MixArgs& a, const MixShape& m, MixLayout lay, int prec,
+                          const std::string& name) {
     Step s;
     s.fn = fn;
-    s.grid = dim3((unsigned)gx, 1, 1);
-    s.block = dim3((unsigned)threads, 1, 1);
-    s.lds_bytes = lds;
-    s.arg.resize(sizeof(GArgs));
-    std::memcpy(s.arg.data(), &g, sizeof(GArgs));
-    s.in_field = (int)(offsetof(GArgs, k) + offsetof(KArgs, in));
-    s.out_field = (int)(offsetof(GArgs, k) + offsetof(KArgs, out));
-    s.nt_field = (int)(offsetof(GArgs, k) + offsetof(KArgs, nt));
+    s.grid = dim3((unsigned)((a.k.count + m.g - 1) / m.g), 1, 1);
+    s.block = dim3((unsigned)m.threads, 1, 1);
+    s.lds_bytes = m.lds;
+    s.arg.resize(sizeof(MixArgs));
+    std::memcpy(s.arg.data(), &a, sizeof(MixArgs));
+    s.in_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, in));
+    s.out_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, out));
+    s.nt_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, nt));
+    s.nt_mask = mix_nt_mask(m, a, lay, prec);
     s.name = name;
     return s;
 }
@@ -689,17 +755,13 @@ static int emit_gen_single(Plan& p, int di, const AxisJob& j, std::string& algo)
     }
     if (!gen_single_fits(prec, j.n, var == VAR_ROW))
         return set_error(AFFT_ERR_NOT_IMPLEMENTED, "mixed radix: length too large for one pass on this layout");
-    GArgs g{};
-    int tpt, lds, threads, rc;
-    bool ipg = false;
-    // strided columns above 128 points (16 threads or more a column) on the
-    // in-place kernel; below, its separate store phase costs more than the
-    // LDS it saves (the 3-point axis of 3 x 5000 x 7: 2.7 % slower)
-    if ((rc = gen_args(p, j.n, var == VAR_ROW, g, &tpt, &lds, &threads, var == VAR_COL && j.n > 128 ? &ipg : nullptr)))
-        return rc;
-    const bool ip = var == VAR_ROW && gen_use_ip(j.n, prec);
-    const void* fn = ip ? gen_ip_kernel(prec, dir) : ipg ? gen_ipg_kernel(prec, var, dir) : gen_kernel(prec, var, dir);
-    if ((rc = prep_dynamic_lds(fn, lds))) return rc;
+    const MixLayout lay = var == VAR_ROW ? MIX_ROWS : MIX_COLS;
+    MixArgs g{};
+    MixShape m;
+    int rc = mix_args(p, j.n, lay, count, slices, g, m);
+    if (rc) return rc;
+    const void* fn = mix_kernel(prec, var, dir);
+    if ((rc = prep_dynamic_lds(fn, m.lds))) return rc;
     g.k.count = count;
     g.k.in_cd = j.in_cd;
     g.k.out_cd = j.out_cd;
@@ -708,8 +770,7 @@ static int emit_gen_single(Plan& p, int di, const AxisJob& j, std::string& algo)
     g.k.in_bd = in_bd;
     g.k.out_bd = out_bd;
     g.k.scale = j.scale;
-    const int G = threads / tpt;
-    Step s = make_gen_step(fn, g, (count + G - 1) / G, lds, threads, "gen" + std::to_string(j.n));
+    Step s = make_mix_step(fn, g, m, lay, prec, "mix" + std::to_string(j.n));
     s.in_role = j.in_role;
     s.out_role = j.out_role;
     s.in_off = j.in_off;
@@ -790,23 +851,22 @@ static int emit_gen_fourstep(Plan& p, int di, const AxisJob& j, std::string& alg
     // kernel of that length, the other factor on the runtime passes.
     const KernelInfo* ka = (is_pow2(n1) && n1 >= 2) ? find_kernel(prec, (int)n1, VAR_4A, dir) : nullptr;
     const KernelInfo* kb = (is_pow2(n2) && n2 >= 2) ? find_kernel(prec, (int)n2, VAR_4B, dir) : nullptr;
-    GArgs ga{}, gb{};
-    int tpa = 1, ldsa = 0, tha = 1, tpb = 1, ldsb = 0, thb = 1;
-    bool ipa = false, ipb = false;
+    MixArgs ga{}, gb{};
+    MixShape ma, mb;
     if (ka) {
         if ((rc = schedule_twiddles(p, ka, &ga.k.tw))) return rc;
-    } else if ((rc = gen_args(p, n1, false, ga, &tpa, &ldsa, &tha, &ipa))) {
+    } else if ((rc = mix_args(p, n1, MIX_COLS, n2, cc, ga, ma))) {
         return rc;
     }
     if (kb) {
         if ((rc = schedule_twiddles(p, kb, &gb.k.tw))) return rc;
-    } else if ((rc = gen_args(p, n2, false, gb, &tpb, &ldsb, &thb, &ipb))) {
+    } else if ((rc = mix_args(p, n2, MIX_TROWS, n1, cc, gb, mb))) {
         return rc;
     }
     if ((rc = split_twiddles(p, prec, j.n, &ga.k.tw4_shift, &ga.k.tw4_lo, &ga.k.tw4_hi))) return rc;
-    const void* fa = ka ? ka->fn : ipa ? gen_ipg_kernel(prec, VAR_4A, dir) : gen_kernel(prec, VAR_4A, dir);
-    const void* fb = kb ? kb->fn : ipb ? gen_ipg_kernel(prec, VAR_4B, dir) : gen_kernel(prec, VAR_4B, dir);
-    if ((!ka && (rc = prep_dynamic_lds(fa, ldsa))) || (!kb && (rc = prep_dynamic_lds(fb, ldsb)))) return rc;
+    const void* fa = ka ? ka->fn : mix_kernel(prec, VAR_4A, dir);
+    const void* fb = kb ? kb->fn : mix_kernel(prec, VAR_4B, dir);
+    if ((!ka && (rc = prep_dynamic_lds(fa, ma.lds))) || (!kb && (rc = prep_dynamic_lds(fb, mb.lds)))) return rc;
     ga.k.tw4_L = j.n;
     ga.k.count = n2;
     ga.k.in_cd = 1; ga.k.in_nd = n2; ga.k.out_cd = 1; ga.k.out_nd = n2;
@@ -816,22 +876,21 @@ static int emit_gen_fourstep(Plan& p, int di, const AxisJob& j, std::string& alg
     gb.k.in_cd = n2; gb.k.in_nd = 1; gb.k.in_bd = j.n;
     gb.k.out_cd = 1; gb.k.out_nd = n1;
     gb.k.scale = j.scale;
-    const int Ga = tha / tpa, Gb = thb / tpb;
     for (int64_t y = 0; y < j.slices; ++y) {
         for (int64_t c0 = 0; c0 < j.count; c0 += cc) {
             const int64_t cnt = std::min(cc, j.count - c0);
-            GArgs a2 = ga, b2 = gb;
+            MixArgs a2 = ga, b2 = gb;
             a2.k.in_bd = j.in_cd;
             b2.k.out_bd = j.out_cd;
             Step sa = ka ? make_step(ka, a2.k, (n2 + ka->tpb - 1) / ka->tpb, 1, "4stepA")
-                         : make_gen_step(fa, a2, (n2 + Ga - 1) / Ga, ldsa, tha, "gen4A");
+                         : make_mix_step(fa, a2, ma, MIX_COLS, prec, "mix4A");
             sa.in_role = j.in_role;
             sa.in_off = j.in_off + (y * j.in_bd + c0 * j.in_cd) * es;
             sa.out_role = ROLE_TMP0;
             sa.out_off = 0;
             push_sliced(p.steps[di], sa, cnt, j.in_cd * es, j.n * es);
             Step sb = kb ? make_step(kb, b2.k, (n1 + kb->tpb - 1) / kb->tpb, 1, "4stepB")
-                         : make_gen_step(fb, b2, (n1 + Gb - 1) / Gb, ldsb, thb, "gen4B");
+                         : make_mix_step(fb, b2, mb, MIX_TROWS, prec, "mix4B");
             sb.in_role = ROLE_TMP0;
             sb.in_off = 0;
             sb.out_role = j.out_role;
@@ -1654,6 +1713,7 @@ int build_plan(Plan& p) {
             if (st.out_role != ROLE_DST || st.nt_field < 0) continue;
             int flags = NT_STORE;
             if (st.in_role == ROLE_SRC && ib >= kStreamOutBytes) flags |= NT_LOAD;
+            flags &= st.nt_mask;
             std::memcpy(st.arg.data() + st.nt_field, &flags, sizeof(int));
         }
     }

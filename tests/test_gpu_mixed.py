@@ -1,0 +1,66 @@
+"""The composite-radix runtime kernel (kmix.hpp) where its launch shapes have
+edges: every radix alone, groups that leave a partial block, several
+butterflies a thread, prime-power and longest lengths, in place, strided
+columns, and four-step factors of a single pass; against the oracle, within
+the library's budgets (helpers.c64_tol, C128_TOL)."""
+import numpy as np
+import pytest
+
+import algofft_hip as A
+from algofft_hip import synth
+import pyoracle as O
+from helpers import C128_TOL, c64_tol, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+PRECS = [(A.COMPLEX64, np.complex64), (A.COMPLEX128, np.complex128)]
+
+
+def _tol(prec, n):
+    return c64_tol(n) if prec == A.COMPLEX64 else C128_TOL
+
+
+# one pass (3 .. 20), two and three passes, powers of one prime, the longest
+# rows of either precision
+ROWS = [3, 5, 6, 7, 9, 10, 12, 14, 15, 18, 20, 21, 24, 28, 54, 175, 360, 525, 686, 2187, 2401, 3125, 7938, 8100]
+
+
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n", ROWS + [14406, 15625, 16200, 16384 - 256])
+def test_rows_with_partial_groups(ctx, n, prec, dt):
+    if prec == A.COMPLEX128 and n > 8192:
+        pytest.skip("longer complex128 rows take the four-step route")
+    batch = 67 if n < 1000 else 3
+    x = synth.uniform_complex(7 * n, (batch, n), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch) as p:
+        assert p.describe() == f"hip_mixed{n}r"
+        got = np.empty_like(x)
+        p.forward(got, x)
+        back = got.copy()
+        p.inverse(back, back)   # in place
+    assert rel_l2(got, O.fft_batch(x.astype(np.complex128))) <= _tol(prec, n)
+    assert rel_l2(back, O.fft_batch(got.astype(np.complex128), inverse=True)) <= _tol(prec, n)
+
+
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n,cols", [(6, 1), (20, 5), (175, 33), (360, 17), (1200, 7), (2401, 3), (4000, 2)])
+def test_strided_columns_with_partial_groups(ctx, n, cols, prec, dt):
+    # columns of a matrix wider than the batch: element stride cols + 2
+    w = cols + 2
+    buf = synth.uniform_complex(n + cols, (n, w), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=cols, istride=w, idist=1, ostride=w, odist=1) as p:
+        out = np.zeros_like(buf)
+        p.forward(out.ravel(), buf.ravel())
+    ref = O.fft_batch(np.ascontiguousarray(buf[:, :cols].T).astype(np.complex128)).T
+    assert rel_l2(out[:, :cols], ref) <= _tol(prec, n)
+
+
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n,split", [(18 * 15, 18), (20 * 20, 20), (12 * 343, 343), (9 * 175, 9), (4050, 2025)])
+def test_fourstep_single_pass_factors(ctx, n, split, prec, dt):
+    x = synth.uniform_complex(3 * n, (3, n), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=3, strategy=A.STRATEGY_SIXSTEP, split=split) as p:
+        assert p.describe() == f"hip_mixed4step{split}x{n // split}"
+        got = np.empty_like(x)
+        p.forward(got, x)
+    assert rel_l2(got, O.fft_batch(x.astype(np.complex128))) <= _tol(prec, n)
