@@ -106,6 +106,13 @@ struct Plan {
     int in_esize[2] = {0, 0};       // bytes per element of each side
     int out_esize[2] = {0, 0};
     std::vector<Step> steps[2];     // [0] forward, [1] inverse
+    // Steps of a direction whose first launch may not write over its input
+    // while other blocks still read it (fused real rows, whose two sides have
+    // different row lengths): the input is copied to WORK2 first.  Used when
+    // the caller's src and dst overlap (alias_steps_for); empty otherwise.
+    std::vector<Step> alias_steps[2];
+    bool alias_same_ok[2] = {false, false};   // src == dst is safe without the copy
+    size_t alias_bytes[2] = {0, 0};           // WORK2 bytes the copy needs
     std::vector<void*> owned;       // device tables
     size_t tmp_bytes[NTMP] = {0, 0, 0, 0};
     void* tmp[NTMP] = {nullptr, nullptr, nullptr, nullptr};
@@ -162,9 +169,12 @@ bool parse_strategy(const std::string& algo, Candidate* c);
 // Predicted log-runtimes of candidates (GPU inference); 0 on success.
 int mlp_predict_host(Mlp* m, const float* x, int64_t n, float* y);
 int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s);
-// The steps of direction di (0 forward, 1 inverse) with explicit workspace
-// buffers; allocates nothing and records no event.
-int launch_steps(Plan& p, int di, void* dst, const void* src, void* const* tmp, hipStream_t s);
+// Steps to run for these buffers: the direction's own, or its aliasing ones
+// where src and dst overlap (the plan's WORK2 size is raised to what they need).
+std::vector<Step>& steps_for(Plan& p, int di, const void* dst, const void* src);
+// Enqueues steps with explicit workspace buffers; allocates nothing and
+// records no event.
+int launch_steps(std::vector<Step>& steps, void* dst, const void* src, void* const* tmp, hipStream_t s);
 // Device address of the static scratch array of afft_plan_exec_device_noalloc
 // on `device`, looked up once per device (noalloc.hip).
 int noalloc_scratch(int device, void** out);

@@ -24,4 +24,9 @@ const void* mix_kernel(int prec, int var, int dir) {
     return cols ? mix_kernel_c128_cols(var, dir) : mix_kernel_c128_rows(var, dir);
 }
 
+const void* mix_real_kernel_c64(int dir);
+const void* mix_real_kernel_c128(int dir);
+
+const void* mix_real_kernel(int prec, int dir) { return prec ? mix_real_kernel_c128(dir) : mix_real_kernel_c64(dir); }
+
 }  // namespace afft

@@ -80,20 +80,21 @@ int afft_plan_exec_device_noalloc(afft_plan p, int direction, void* dst, const v
         return set_error(AFFT_ERR_INVALID_ARGUMENT, "direction must be -1 or +1");
     const int di = direction == AFFT_INVERSE ? 1 : 0;
     if (p->steps[di].empty()) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "direction not available for this plan kind");
+    std::lock_guard<std::mutex> lock(p->mu);
+    std::vector<Step>& steps = steps_for(*p, di, dst, src);
     size_t off[NTMP];
     const size_t need = carve(*p, off);
     if (need > kNoAllocScratchBytes)
         return set_error(AFFT_ERR_INVALID_LENGTH, "plan needs " + std::to_string(need) +
                                                       " bytes of scratch; the static scratch holds " +
                                                       std::to_string(kNoAllocScratchBytes));
-    std::lock_guard<std::mutex> lock(p->mu);
     void* base = nullptr;
     int rc = noalloc_scratch(p->ctx->device, &base);
     if (rc) return rc;
     AFFT_HIP(hipSetDevice(p->ctx->device));
     void* tmp[NTMP];
     for (int t = 0; t < NTMP; ++t) tmp[t] = p->tmp_bytes[t] ? (char*)base + off[t] : nullptr;
-    rc = launch_steps(*p, di, dst, src, tmp, stream ? (hipStream_t)stream : p->stream);
+    rc = launch_steps(steps, dst, src, tmp, stream ? (hipStream_t)stream : p->stream);
     if (rc == AFFT_OK) clear_error();
     return rc;
 }

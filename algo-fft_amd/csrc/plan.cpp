@@ -1372,6 +1372,7 @@ static int emit_nd_axes(Plan& p, int di, int rank, const int64_t* cd, const std:
 }
 
 const void* rpost_kernel(int prec, int dir);
+const void* mix_real_kernel(int prec, int dir);
 
 // Real rows of n reals (h = n/2 complex points): `rows` rows, row r of slice y
 // at y*bd + r*rd (complex elements of each side; the real side counts the
@@ -1421,6 +1422,43 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
             s.out_off = y * out_bd * es;
             s.name = di ? "c2r" : "r2c";
             p.steps[di].push_back(s);
+        }
+        if (!algo.empty()) algo += "+";
+        algo += (di ? "c2r" : "r2c") + std::to_string(n);
+        return AFFT_OK;
+    }
+    // smooth h held in LDS: the runtime-radix kernel with the recombination
+    if (h >= 2 && !is_pow2(h) && !smooth_schedule(h).empty() && h <= gen_row_cap(prec)) {
+        MixRealArgs a{};
+        MixShape m;
+        if ((rc = mix_args(p, h, MIX_ROWS, rows, slices, a.m, m))) return rc;
+        const void* fn = mix_real_kernel(prec, dir);
+        if ((rc = prep_dynamic_lds(fn, m.lds))) return rc;
+        a.wk = wk;
+        a.m.k.count = rows;
+        a.m.k.in_cd = in_rd;
+        a.m.k.out_cd = out_rd;
+        a.m.k.scale = di ? scale / (double)h : scale;
+        for (int64_t y = 0; y < slices; ++y) {
+            Step s;
+            s.fn = fn;
+            s.grid = dim3((unsigned)((rows + m.g - 1) / m.g), 1, 1);
+            s.block = dim3((unsigned)m.threads, 1, 1);
+            s.lds_bytes = m.lds;
+            s.arg.resize(sizeof(MixRealArgs));
+            std::memcpy(s.arg.data(), &a, sizeof(MixRealArgs));
+            s.in_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, in));
+            s.out_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, out));
+            s.in_role = in_role;
+            s.out_role = out_role;
+            s.in_off = y * in_bd * es;
+            s.out_off = y * out_bd * es;
+            s.name = di ? "mixc2r" : "mixr2c";
+            p.steps[di].push_back(s);
+        }
+        if (in_role == ROLE_SRC && out_role == ROLE_DST) {
+            p.alias_same_ok[di] = in_rd == out_rd && (slices == 1 || in_bd == out_bd);
+            p.alias_bytes[di] = (size_t)p.in_elems[di] * p.in_esize[di];
         }
         if (!algo.empty()) algo += "+";
         algo += (di ? "c2r" : "r2c") + std::to_string(n);
@@ -1644,11 +1682,23 @@ static int build_plan_steps(Plan& p) {
     return AFFT_OK;
 }
 
-// Enqueues the steps of direction di on s, with the roles resolved to src,
-// dst and the workspace buffers tmp[0 .. NTMP).
-int launch_steps(Plan& p, int di, void* dst, const void* src, void* const* tmp, hipStream_t s) {
+std::vector<Step>& steps_for(Plan& p, int di, const void* dst, const void* src) {
+    if (p.alias_steps[di].empty() || (src == dst && p.alias_same_ok[di])) return p.steps[di];
+    const char* s0 = (const char*)src;
+    const char* d0 = (const char*)dst;
+    const bool apart = s0 + (size_t)p.in_elems[di] * p.in_esize[di] <= d0 ||
+                       d0 + (size_t)p.out_elems[di] * p.out_esize[di] <= s0;
+    if (apart) return p.steps[di];
+    size_t& w = p.tmp_bytes[ROLE_WORK2 - 2];
+    w = std::max({w, p.alias_bytes[0], p.alias_bytes[1]});
+    return p.alias_steps[di];
+}
+
+// Enqueues steps on s, with the roles resolved to src, dst and the workspace
+// buffers tmp[0 .. NTMP).
+int launch_steps(std::vector<Step>& steps, void* dst, const void* src, void* const* tmp, hipStream_t s) {
     void* base[ROLE_COUNT] = {const_cast<void*>(src), dst, tmp[0], tmp[1], tmp[2], tmp[3]};
-    for (Step& st : p.steps[di]) {
+    for (Step& st : steps) {
         char* ip = (char*)base[st.in_role] + st.in_off;
         char* op = (char*)base[st.out_role] + st.out_off;
         std::memcpy(st.arg.data() + st.in_field, &ip, sizeof(void*));
@@ -1667,6 +1717,7 @@ int launch_steps(Plan& p, int di, void* dst, const void* src, void* const* tmp, 
 // touched.
 int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
     const int di = dir == AFFT_INVERSE ? 1 : 0;
+    std::vector<Step>& steps = steps_for(p, di, dst, src);
     bool ws = false;
     for (int t = 0; t < NTMP; ++t) {
         if (!p.tmp_bytes[t]) continue;
@@ -1683,7 +1734,7 @@ int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
             if (p.ws_used && p.ws_stream != s) AFFT_HIP(hipStreamWaitEvent(s, p.ws_done, 0));
         }
     }
-    int rc = launch_steps(p, di, dst, src, p.tmp, s);
+    int rc = launch_steps(steps, dst, src, p.tmp, s);
     if (rc) return rc;
     if (ws) {
         AFFT_HIP(hipEventRecord(p.ws_done, s));
@@ -1702,9 +1753,25 @@ int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
 // streaming loads alone lose.
 constexpr size_t kStreamOutBytes = size_t(128) << 20;
 
+static void build_alias_steps(Plan& p) {
+    const int prec = p.desc.precision;
+    for (int di = 0; di < 2; ++di) {
+        if (!p.alias_bytes[di]) continue;
+        Step c = make_copy(prec, 1, (int64_t)(p.alias_bytes[di] / (prec ? 16 : 8)), 0, 1, 0, 1, 1.0);
+        c.in_role = ROLE_SRC;
+        c.out_role = ROLE_WORK2;
+        p.alias_steps[di].push_back(c);
+        for (Step s : p.steps[di]) {
+            if (s.in_role == ROLE_SRC) s.in_role = ROLE_WORK2;
+            p.alias_steps[di].push_back(s);
+        }
+    }
+}
+
 int build_plan(Plan& p) {
     int rc = build_plan_steps(p);
     if (rc) return rc;
+    build_alias_steps(p);
     for (int di = 0; di < 2; ++di) {
         const size_t ob = (size_t)p.out_elems[di] * p.out_esize[di];
         const size_t ib = (size_t)p.in_elems[di] * p.in_esize[di];

@@ -5,6 +5,7 @@ columns, and four-step factors of a single pass; against the oracle, within
 the library's budgets (helpers.c64_tol, C128_TOL)."""
 import numpy as np
 import pytest
+import torch
 
 import algofft_hip as A
 from algofft_hip import synth
@@ -64,3 +65,50 @@ def test_fourstep_single_pass_factors(ctx, n, split, prec, dt):
         got = np.empty_like(x)
         p.forward(got, x)
     assert rel_l2(got, O.fft_batch(x.astype(np.complex128))) <= _tol(prec, n)
+
+
+REAL_H = [3, 5, 9, 12, 18, 20, 21, 50, 175, 525, 960, 2401, 5400, 7938]
+
+
+@pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
+@pytest.mark.parametrize("h", REAL_H + [16200])
+def test_real_rows(ctx, h, prec):
+    if prec == A.COMPLEX128 and h > 8192:
+        pytest.skip("longer complex128 rows run unfused")
+    rdt = np.float32 if prec == A.COMPLEX64 else np.float64
+    cdt = np.complex64 if prec == A.COMPLEX64 else np.complex128
+    n, batch = 2 * h, 67 if h < 1000 else 3
+    x = synth.uniform_real(h, (batch, n), rdt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, kind=A.R2C, batch=batch) as p:
+        X = np.empty((batch, h + 1), cdt)
+        p.forward(X, x)
+        y = np.empty_like(x)
+        p.inverse(y, X)
+    assert rel_l2(X, O.rfft(x.astype(np.float64))) <= _tol(prec, n)
+    assert rel_l2(y, O.irfft(X.astype(np.complex128), n)) <= _tol(prec, n)
+
+
+@pytest.mark.parametrize("dims", [(50,), (1050,), (6, 50)])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_real_rows_over_their_own_input(ctx, dims, noalloc):
+    """Packed real plans with dst at src: a row's output lies over the next
+    row's input, so the input is copied first."""
+    batch, n = 37, dims[-1]
+    rows = batch * int(np.prod(dims[:-1], dtype=np.int64))
+    x = synth.uniform_real(n, (batch,) + dims, np.float32)
+    X = np.fft.rfftn(x.astype(np.float64), axes=tuple(range(1, len(dims) + 1)))
+    buf = torch.zeros(rows * (n // 2 + 1) * 2, dtype=torch.float32, device="cuda")
+    s = torch.cuda.Stream()
+    import ctypes
+    fn = A.lib().afft_plan_exec_device_noalloc if noalloc else A.lib().afft_plan_exec_device
+    with A.Plan.from_desc(ctx, dims, kind=A.R2C, batch=batch) as p:
+        buf[:x.size] = torch.from_numpy(x.ravel()).cuda()
+        torch.cuda.synchronize()
+        for d in (A.FORWARD, A.INVERSE):
+            A.check(fn(p.h, d, ctypes.c_void_p(buf.data_ptr()), ctypes.c_void_p(buf.data_ptr()),
+                       ctypes.c_void_p(s.cuda_stream)))
+            s.synchronize()
+            if d == A.FORWARD:
+                got = torch.view_as_complex(buf.view(-1, 2)).cpu().numpy().reshape(X.shape)
+                assert rel_l2(got, X) <= c64_tol(x[0].size)
+    assert rel_l2(buf[:x.size].cpu().numpy().reshape(x.shape), x) <= 2 * c64_tol(x[0].size)
