@@ -140,6 +140,11 @@ int build_plan(Plan& p);
 int upload_table(Plan& p, const void* host, size_t bytes, const void** dev);
 std::vector<int> smooth_schedule(int64_t n);   // empty unless 2/3/5/7-smooth
 int64_t next_pow2(int64_t n);
+struct MixArgs;
+// Runtime mixed-radix rows: the passes, twiddles (owned by p) and launch shape
+// of `count` transforms of n points, n 7-smooth and at most gen_row_cap.
+int mix_row_launch(Plan& p, int64_t n, int64_t count, MixArgs& a, int* threads, int* lds);
+int prep_dynamic_lds(const void* fn, int lds);
 struct BlueTables {
     const void* chirp = nullptr;                 // n entries, forward sign
     const void* filt[2] = {nullptr, nullptr};    // [fwd, inv], m entries, 1/m folded in

@@ -11,12 +11,21 @@
 // the padding kernel does on the fly.  Real convolution (ConvolveReal) pads
 // real rows to an even 7-smooth F, runs R2C on both, multiplies the half
 // spectra and returns through C2R.
+//
+// Where F points (F/2 complex ones for real rows) fit in LDS all of that is
+// one launch (kconv.hpp).  Longer rows, and calls whose output lies over an
+// input, run pad, transform, product, transform and crop as launches of their
+// own through the work buffers.
 #include <algorithm>
 #include <cstring>
 
 #include "afft_internal.hpp"
+#include "kconv.hpp"
 
 namespace afft {
+
+const void* mix_conv_kernel_c64(bool real);
+const void* mix_conv_kernel_c128(bool real);
 
 struct PadArgs {
     const void* src;
@@ -97,6 +106,9 @@ struct afft_conv_s {
     afft_plan inv = nullptr;  // inverse: the batch product rows
     void* work = nullptr;     // 2 * batch * f complex (real mode: 2 * batch * f reals)
     void* spec = nullptr;     // real mode: 2 * batch * (f/2 + 1) complex spectra
+    const void* fn = nullptr; // one-launch form, if F fits
+    MixConvArgs fused{};
+    int threads = 0, lds = 0;
     hipStream_t stream = nullptr;
     std::mutex mu;
     ~afft_conv_s() {
@@ -118,6 +130,37 @@ static int64_t smooth_at_least(int64_t n, bool even = false) {
             while (t % q == 0) t /= q;
         if (t == 1) return m;
     }
+}
+
+// The one-launch form of c, with its tables owned by c->plan.
+static int prepare_fused(afft_conv_s& c) {
+    const bool real = c.mode == AFFT_CONV_REAL;
+    const int64_t n = real ? c.f / 2 : c.f;
+    if (n < 2 || n > gen_row_cap(c.prec)) return AFFT_OK;
+    Plan& p = *c.plan;
+    MixConvArgs& g = c.fused;
+    int rc = mix_row_launch(p, n, c.batch, g.m, &c.threads, &c.lds);
+    if (rc) return rc;
+    if (real) {
+        std::vector<double> w(2 * (n / 2 + 1));
+        for (int64_t k = 0; k <= n / 2; ++k) root_of_unity(k, c.f, &w[2 * k], &w[2 * k + 1]);
+        std::vector<float> f(w.begin(), w.end());
+        rc = c.prec ? upload_table(p, w.data(), w.size() * 8, &g.wk) : upload_table(p, f.data(), f.size() * 4, &g.wk);
+        if (rc) return rc;
+    }
+    g.na = (int)c.na;
+    g.nb = (int)c.nb;
+    g.len = (int)c.len;
+    g.revconj = c.mode == AFFT_CONV_CORRELATE;
+    g.m.k.scale = 1.0 / (double)n;
+    const void* fn = c.prec ? mix_conv_kernel_c128(real) : mix_conv_kernel_c64(real);
+    if ((rc = prep_dynamic_lds(fn, c.lds))) return rc;
+    c.fn = fn;
+    return AFFT_OK;
+}
+
+static bool overlap(const void* p, size_t pn, const void* q, size_t qn) {
+    return (const char*)p < (const char*)q + qn && (const char*)q < (const char*)p + pn;
 }
 
 static int launch(const void* fn, int64_t total, void* args, hipStream_t s) {
@@ -161,6 +204,7 @@ int afft_conv_create(afft_context ctx, int precision, int64_t na, int64_t nb, in
     int rc = afft_plan_create_desc(ctx, &d, &c->plan);
     d.batch = batch;
     if (!rc) rc = afft_plan_create_desc(ctx, &d, &c->inv);
+    if (!rc) rc = prepare_fused(*c);
     hipError_t e = hipSuccess;
     const size_t ce = precision ? 16 : 8;
     if (!rc) e = hipMalloc(&c->work, (size_t)(2 * batch * c->f) * (real ? ce / 2 : ce));
@@ -185,6 +229,18 @@ int afft_conv_exec(afft_conv c, void* dst, const void* a, const void* b, void* s
     std::lock_guard<std::mutex> l(c->mu);
     AFFT_HIP(hipSetDevice(c->ctx->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
+    const size_t eb = (size_t)(c->prec ? 16 : 8) / (c->mode == AFFT_CONV_REAL ? 2 : 1) * c->batch;
+    if (c->fn && !overlap(dst, eb * c->len, a, eb * c->na) && !overlap(dst, eb * c->len, b, eb * c->nb)) {
+        MixConvArgs g = c->fused;
+        g.dst = dst;
+        g.a = a;
+        g.b = b;
+        void* args[] = {&g};
+        const int64_t blocks = (c->batch + g.m.g - 1) / g.m.g;
+        AFFT_HIP(hipLaunchKernel(c->fn, dim3((unsigned)blocks), dim3((unsigned)c->threads), args, (size_t)c->lds, s));
+        clear_error();
+        return AFFT_OK;
+    }
     if (c->mode == AFFT_CONV_REAL) {
         // real rows padded to f, half spectra of f/2 + 1, product, C2R, crop
         const int rs = c->prec ? 8 : 4, cs = 2 * rs;

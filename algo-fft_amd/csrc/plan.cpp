@@ -694,6 +694,15 @@ static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t sl
     return upload_table(p, tw.data(), tw.size() * 8, &a.k.tw);
 }
 
+int mix_row_launch(Plan& p, int64_t n, int64_t count, MixArgs& a, int* threads, int* lds) {
+    MixShape m;
+    const int rc = mix_args(p, n, MIX_ROWS, count, 1, a, m);
+    a.k.count = count;
+    *threads = m.threads;
+    *lds = m.lds;
+    return rc;
+}
+
 // Non-temporal accesses pay only where a wave covers whole lines: rows whose
 // first and last passes run at least 512 contiguous bytes (complex64 60
 // points 0.259 -> 0.200 ms without them, 525 0.224 -> 0.204; 960 0.183 ->
@@ -729,7 +738,7 @@ static Step make_mix_step(const void* fn, const MixArgs& a, const MixShape& m, M
     return s;
 }
 
-static int prep_dynamic_lds(const void* fn, int lds) {
+int prep_dynamic_lds(const void* fn, int lds) {
     if (lds > 65536) AFFT_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     return AFFT_OK;
 }

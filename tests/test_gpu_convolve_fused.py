@@ -1,0 +1,80 @@
+"""The one-launch convolution (kconv.hpp) over batches: its shortest and
+longest padded lengths, the first beyond them (the launches of their own),
+partial groups, odd and one-element rows, and an output over an input;
+against FP64 FFT convolution, within the library's budgets."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import algofft_hip as A
+from algofft_hip import synth
+from helpers import C128_TOL, c64_tol, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+# (na, nb, batch): complex cap 16384 (complex64) / 8192 padded points, real
+# rows twice that
+SHAPES = [(1, 1, 5), (2, 1, 3), (3, 4, 67), (7, 5, 33), (100, 29, 41), (777, 65, 32), (1009, 1009, 5), (4000, 93, 3),
+          (5000, 3193, 2), (8000, 400, 2), (9000, 7300, 2), (16000, 16001, 1), (20000, 13000, 1)]
+
+
+def _ref(a, b, mode):
+    if mode == A.CONV_CORRELATE:
+        b = np.conj(b[:, ::-1])
+    n = a.shape[1] + b.shape[1] - 1
+    f = 1 << int(np.ceil(np.log2(max(n, 2))))
+    y = np.fft.ifft(np.fft.fft(a, f, axis=1) * np.fft.fft(b, f, axis=1), axis=1)[:, :n]
+    return y.real if mode == A.CONV_REAL else y
+
+
+def _run(ctx, prec, mode, na, nb, batch, dst, a, b):
+    h = ctypes.c_void_p()
+    A.check(A.lib().afft_conv_create(ctx.h, prec, na, nb, batch, mode, ctypes.byref(h)))
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        A.check(A.lib().afft_conv_exec(h, ctypes.c_void_p(dst.data_ptr()), ctypes.c_void_p(a.data_ptr()),
+                                       ctypes.c_void_p(b.data_ptr()), ctypes.c_void_p(s.cuda_stream)))
+        s.synchronize()
+    finally:
+        A.check(A.lib().afft_conv_destroy(h))
+
+
+def _data(prec, mode, na, nb, batch):
+    wide = prec == A.COMPLEX128
+    if mode == A.CONV_REAL:
+        dt = np.float64 if wide else np.float32
+        return synth.uniform_real(na, (batch, na), dt), synth.uniform_real(nb + 7, (batch, nb), dt)
+    dt = np.complex128 if wide else np.complex64
+    return synth.uniform_complex(na, (batch, na), dt), synth.uniform_complex(nb + 7, (batch, nb), dt)
+
+
+@pytest.mark.parametrize("na,nb,batch", SHAPES)
+@pytest.mark.parametrize("mode", [A.CONV_LINEAR, A.CONV_CORRELATE, A.CONV_REAL])
+@pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
+def test_batched_convolution(ctx, na, nb, batch, mode, prec):
+    a, b = _data(prec, mode, na, nb, batch)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    out = torch.empty((batch, na + nb - 1), dtype=ta.dtype, device="cuda")
+    _run(ctx, prec, mode, na, nb, batch, out, ta, tb)
+    tol = c64_tol(na + nb) if prec == A.COMPLEX64 else C128_TOL
+    wide = np.float64 if mode == A.CONV_REAL else np.complex128
+    assert rel_l2(out.cpu().numpy(), _ref(a.astype(wide), b.astype(wide), mode)) <= tol
+
+
+@pytest.mark.parametrize("mode", [A.CONV_LINEAR, A.CONV_REAL])
+@pytest.mark.parametrize("over", ["a", "b"])
+def test_output_over_an_input(ctx, mode, over):
+    na, nb, batch = 300, 45, 37
+    a, b = _data(A.COMPLEX64, mode, na, nb, batch)
+    big, small = (a, b) if over == "a" else (b, a)
+    buf = torch.zeros(batch * (na + nb - 1), dtype=torch.from_numpy(a).dtype, device="cuda")
+    buf[:big.size] = torch.from_numpy(big.ravel()).cuda()
+    t = torch.from_numpy(small).cuda()
+    ta, tb = (buf, t) if over == "a" else (t, buf)
+    _run(ctx, A.COMPLEX64, mode, na, nb, batch, buf, ta, tb)
+    wide = np.float64 if mode == A.CONV_REAL else np.complex128
+    got = buf.cpu().numpy().reshape(batch, na + nb - 1)
+    assert rel_l2(got, _ref(a.astype(wide), b.astype(wide), mode)) <= c64_tol(na + nb)
