@@ -43,6 +43,7 @@ struct KArgs {
     const void* fvec;
     long long flen;
     int nt;                  // NT_STORE / NT_LOAD: non-temporal output stores / input loads
+    int xcd;                 // column layouts of k_fft: blocks in XCD order (xcd_block)
 };
 
 enum { FUSE_NONE = 0, FUSE_CHIRP_IN = 1, FUSE_MUL_OUT = 2, FUSE_CROP_OUT = 3 };
@@ -79,6 +80,19 @@ __device__ __forceinline__ cx<T> tw4(const KArgs& a, long long m) {
     return cmul(lo[m & mask], hi[m >> a.tw4_shift]);
 }
 
+// The work item of this block for neighbouring items on one XCD: consecutive
+// blocks go to the 8 XCDs (each with its own L2) in turn; the result is the
+// item of the block's position within its XCD's share (a bijection of the
+// grid).
+__device__ __forceinline__ void xcd_block(unsigned* bx, unsigned* by) {
+    constexpr unsigned XCDS = 8;
+    const unsigned tot = gridDim.x * gridDim.y, lin = *by * gridDim.x + *bx;
+    const unsigned q = tot / XCDS, r = tot % XCDS, x = lin % XCDS;
+    const unsigned nl = x * q + (x < r ? x : r) + lin / XCDS;
+    *by = nl / gridDim.x;
+    *bx = nl - *by * gridDim.x;
+}
+
 template <typename T, class S, int E, int TPB, int VAR, int DIR>
 __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArgs a) {
     using C = KCfg<T, S, E, TPB, VAR>;
@@ -89,9 +103,12 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
     int c, t;
     if constexpr (C::ROWL) { c = tid / TT; t = tid % TT; }
     else { c = tid % TPB; t = tid / TPB; }
-    const long long cg = (long long)blockIdx.x * TPB + c;
+    unsigned bx = blockIdx.x, by = blockIdx.y;
+    if constexpr (VAR != VAR_ROW)
+        if (a.xcd) xcd_block(&bx, &by);
+    const long long cg = (long long)bx * TPB + c;
     const bool act = cg < a.count;
-    const cx<T>* __restrict__ in = (const cx<T>*)a.in + (long long)blockIdx.y * a.in_bd;
+    const cx<T>* __restrict__ in = (const cx<T>*)a.in + (long long)by * a.in_bd;
     const cx<T>* __restrict__ tw = (const cx<T>*)a.tw;
     cx<T> v[E];
 
@@ -138,7 +155,7 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
     }
 
     if constexpr (VAR == VAR_4A) {
-        const long long col = (a.tw4_by_y ? (long long)blockIdx.y : cg) + a.tw4_c0;
+        const long long col = (a.tw4_by_y ? (long long)by : cg) + a.tw4_c0;
         // W_L^{k*col} for k = t + TT*e (k < N and col < L/N, so k*col < L
         // needs no reduction).  Lanes differ in col, so every table load
         // gathers from scattered lines: look up every fourth e and step
@@ -167,7 +184,7 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
         for (int e = 0; e < E; ++e) v[e] = scl(v[e], s);
     }
 
-    cx<T>* __restrict__ out = (cx<T>*)a.out + (long long)blockIdx.y * a.out_bd;
+    cx<T>* __restrict__ out = (cx<T>*)a.out + (long long)by * a.out_bd;
     if constexpr (VAR == VAR_ROW) {
         if (act) {
             cx<T>* dst = out + cg * a.out_cd;
@@ -189,7 +206,7 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
         __syncthreads();
         const int c2 = tid % TPB, t2 = tid / TPB;
         LdsRow<N, C::PADSH> li2(c2);
-        const long long cg2 = (long long)blockIdx.x * TPB + c2;
+        const long long cg2 = (long long)bx * TPB + c2;
         if (cg2 < a.count) {
             const long long nd = a.out_nd;
             if (a.fuse == FUSE_NONE) {

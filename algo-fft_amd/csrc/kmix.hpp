@@ -224,23 +224,13 @@ __global__ void __launch_bounds__(MixCfg<T>::THREADS, MixCfg<T>::WAVES) k_mix(Mi
     int c, t;
     if constexpr (COLL) t = fast_divmod(tid, G, g.divm, &c);
     else c = fast_divmod(tid, TPT, g.divm, &t);
-    // Consecutive blocks go to the 8 XCDs (each with its own L2) in turn, so
-    // neighbouring column groups, which share cache lines unless they start
-    // and end on line boundaries, would be fetched or written by different
-    // L2s.  A block takes the work item of its position within its XCD's
-    // share instead (a bijection of the grid).  Columns of 8 complex64 (half
-    // lines), rows of 512: 1200 points 0.339 -> 0.275 ms, 2000 0.344 ->
+    // Neighbouring column groups share cache lines unless they start and end
+    // on line boundaries: blocks in XCD order keep them in one L2.  Columns
+    // of 8 complex64 (half lines), rows of 512: 1200 points 0.339 -> 0.275 ms, 2000 0.344 ->
     // 0.296; 16 columns, rows of 961: 500 points 0.354 -> 0.266; transposing
     // stores (VAR_4B), rows of 500: 400 points 0.318 -> 0.251.
     unsigned bx = blockIdx.x, by = blockIdx.y;
-    if constexpr (VAR != VAR_ROW) {
-        constexpr unsigned XCDS = 8;
-        const unsigned tot = gridDim.x * gridDim.y, lin = by * gridDim.x + bx;
-        const unsigned q = tot / XCDS, r = tot % XCDS, x = lin % XCDS;
-        const unsigned nl = x * q + (x < r ? x : r) + lin / XCDS;
-        by = nl / gridDim.x;
-        bx = nl - by * gridDim.x;
-    }
+    if constexpr (VAR != VAR_ROW) xcd_block(&bx, &by);
     const long long c0 = (long long)bx * G;
     const bool act = tid < G * TPT && c0 + c < a.count;
     const cx<T>* __restrict__ in = (const cx<T>*)a.in + (long long)by * a.in_bd;
