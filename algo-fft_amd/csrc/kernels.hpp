@@ -17,7 +17,7 @@
 
 namespace afft {
 
-enum { VAR_ROW = 0, VAR_COL = 1, VAR_4A = 2, VAR_4B = 3, VAR_COUNT = 4, VAR_BLUE = 4, VAR_REAL = 5 };
+enum { VAR_ROW = 0, VAR_COL = 1, VAR_4A = 2, VAR_4B = 3, VAR_COUNT = 4, VAR_BLUE = 4, VAR_REAL = 5, VAR_BLUEMID = 6 };
 
 struct KArgs {
     const void* in;
@@ -34,10 +34,9 @@ struct KArgs {
     long long tw4_L;
     long long tw4_c0;        // column index offset of this launch
     int tw4_by_y;            // 1: the four-step column index is blockIdx.y, not c
-    // Bluestein fusion on the four-step passes (runtime, uniform per launch):
+    // Bluestein fusion on the column passes (runtime, uniform per launch):
     //   FUSE_CHIRP_IN (VAR_4A): x[n] * chirp[n] for n < flen, zero beyond
-    //   FUSE_MUL_OUT  (VAR_4B): y[k] * fvec[k]
-    //   FUSE_CROP_OUT (VAR_4B): y[k] * fvec[k] stored only for k < flen
+    //   FUSE_CROP_OUT (VAR_COL): y[k] * fvec[k] stored only for k < flen
     int fuse;
     int fconj;               // use conj(fvec)
     const void* fvec;
@@ -46,7 +45,7 @@ struct KArgs {
     int xcd;                 // column layouts of k_fft: blocks in XCD order (xcd_block)
 };
 
-enum { FUSE_NONE = 0, FUSE_CHIRP_IN = 1, FUSE_MUL_OUT = 2, FUSE_CROP_OUT = 3 };
+enum { FUSE_NONE = 0, FUSE_CHIRP_IN = 1, FUSE_CROP_OUT = 2 };
 
 template <typename T>
 __device__ __forceinline__ cx<T> fvec_at(const void* f, long long i, int conj) {
@@ -195,8 +194,16 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
         if (act) {
             cx<T>* dst = out + cg;
             const long long nd = a.out_nd;
+            if (VAR == VAR_COL && a.fuse == FUSE_CROP_OUT) {
 #pragma unroll
-            for (int e = 0; e < E; ++e) st_out(dst + (long long)(t + TT * e) * nd, v[e], a.nt);
+                for (int e = 0; e < E; ++e) {
+                    const long long k = cg + (long long)(t + TT * e) * nd;
+                    if (k < a.flen) out[k] = cmul(v[e], fvec_at<T>(a.fvec, k, a.fconj));
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < E; ++e) st_out(dst + (long long)(t + TT * e) * nd, v[e], a.nt);
+            }
         }
     } else {  // VAR_4B: re-map through LDS so lanes run along c on the store
         LdsRow<N, C::PADSH> li(c);
@@ -209,17 +216,8 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
         const long long cg2 = (long long)bx * TPB + c2;
         if (cg2 < a.count) {
             const long long nd = a.out_nd;
-            if (a.fuse == FUSE_NONE) {
 #pragma unroll
-                for (int e = 0; e < E; ++e) st_out(out + cg2 + (long long)(t2 + TT * e) * nd, lds[li2(t2 + TT * e)], a.nt);
-            } else {
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    const long long k = cg2 + (long long)(t2 + TT * e) * nd;
-                    const cx<T> y = cmul(lds[li2(t2 + TT * e)], fvec_at<T>(a.fvec, k < a.flen ? k : 0, a.fconj));
-                    if (a.fuse == FUSE_MUL_OUT || k < a.flen) out[k] = y;
-                }
-            }
+            for (int e = 0; e < E; ++e) st_out(out + cg2 + (long long)(t2 + TT * e) * nd, lds[li2(t2 + TT * e)], a.nt);
         }
     }
 }
@@ -273,6 +271,50 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR_ROW>::THREADS)) k_blue
         for (int e = 0; e < E; ++e) {
             const int n = t + TT * e;
             if (n < a.nlog) dst[n] = scl(twmul<DIR>(v[e], chirp[n]), sc);
+        }
+    }
+}
+
+// Middle pass of a Bluestein chain whose M = m1 * m2 is beyond LDS, between
+// the column passes over m1: row k1 of the forward transform's m1 x m2
+// intermediate runs its FFT over n2, the product with the filter (stored
+// row-major as [k1][k2] for k = k1 + m1*k2), the inverse FFT over k2 and the
+// inverse twiddle W_M^{-k1*n2}, in place and contiguous.  The spectrum is
+// never put into natural order, so the chain has three passes and no
+// transposing store (as four four-step passes: complex128 1,000,003 points x 8
+// 0.586 -> 0.384 ms, complex64 100,003 x 64 0.235 -> 0.159, complex128 10,007 x
+// 400 0.359 -> 0.228).  Bound by the column passes' access pattern.
+// in_cd / out_cd: m2; fvec: the filter, 1/M folded in.
+template <typename T, class S, int E, int TPB>
+__global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR_ROW>::THREADS)) k_bluemid(KArgs a) {
+    using C = KCfg<T, S, E, TPB, VAR_ROW>;
+    constexpr int TT = C::TT;
+    __shared__ cx<T> lds[C::LDS_ELEMS];
+    const int tid = threadIdx.x;
+    const int c = tid / TT, t = tid % TT;
+    const long long cg = (long long)blockIdx.x * TPB + c;
+    const bool act = cg < a.count;
+    const cx<T>* __restrict__ src = (const cx<T>*)a.in + (long long)blockIdx.y * a.in_bd + cg * a.in_cd;
+    const cx<T>* __restrict__ filt = (const cx<T>*)a.fvec + cg * a.in_cd;
+    const cx<T>* __restrict__ tw = (const cx<T>*)a.tw;
+    cx<T> v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = act ? src[t + TT * e] : mk<T>(0, 0);
+    LdsRow<S::N, C::PADSH> li(c);
+    core<T, S, E, -1>(v, lds, t, tw, li);
+    if (act) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = cmul(v[e], filt[t + TT * e]);
+    }
+    core<T, S, E, 1, true>(v, lds, t, tw, li);
+    if (act) {
+        cx<T>* dst = (cx<T>*)a.out + (long long)blockIdx.y * a.out_bd + cg * a.out_cd;
+        const cx<T> st = tw4<T>(a, (long long)TT * cg);
+        cx<T> w = mk<T>(1, 0);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            w = e % 4 == 0 ? tw4<T>(a, (long long)(t + TT * e) * cg) : cmul(w, st);
+            dst[t + TT * e] = cmulc(v[e], w);
         }
     }
 }
@@ -467,6 +509,9 @@ struct Registrar {
         if constexpr (VAR == VAR_BLUE) {
             k.fn = (const void*)&k_blue<T, S, E, TPB, DIR>;
             k.kind = KIND_BLUE;
+        } else if constexpr (VAR == VAR_BLUEMID) {
+            k.fn = (const void*)&k_bluemid<T, S, E, TPB>;   // one kernel for both plan directions
+            k.kind = KIND_FFT;
         } else if constexpr (VAR == VAR_REAL) {
             k.fn = (const void*)&k_real<T, S, E, TPB, DIR>;
             k.kind = KIND_REAL;

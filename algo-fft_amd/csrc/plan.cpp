@@ -1073,13 +1073,40 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
         const int64_t m2 = tr_m1 > 0 ? m / tr_m1 : 0;
         const double inv_m = 1.0 / (double)m;   // m is a power of two: exact
         for (int d = 0; d < 2; ++d) filt[d].resize(2 * m);
-        for (int64_t k = 0; k < m; ++k) {
-            const int64_t at = tr_m1 > 0 ? (k % tr_m1) * m2 + k / tr_m1 : k;
-            const int64_t mk_ = (m - k) & (m - 1);
-            filt[0][2 * at] = spec[2 * k] * inv_m;
-            filt[0][2 * at + 1] = spec[2 * k + 1] * inv_m;
-            filt[1][2 * at] = spec[2 * mk_] * inv_m;
-            filt[1][2 * at + 1] = -spec[2 * mk_ + 1] * inv_m;
+        // filt[0][at] = spec[k] / m, filt[1][at] = conj(spec[-k mod m]) / m,
+        // through a buffer where the order changes (runs of 32 points read,
+        // of 256 points written)
+        auto put = [&](const double* f, const double* r, int64_t at) {
+            filt[0][2 * at] = f[0] * inv_m;
+            filt[0][2 * at + 1] = f[1] * inv_m;
+            filt[1][2 * at] = r[0] * inv_m;
+            filt[1][2 * at + 1] = -r[1] * inv_m;
+        };
+        if (tr_m1 > 0) {
+            constexpr int64_t T1 = 32, T2 = 256;
+            std::vector<double> buf(4 * T1 * (T2 + 1));
+            for (int64_t r0 = 0; r0 < tr_m1; r0 += T1) {
+                const int64_t n1 = std::min(T1, tr_m1 - r0);
+                for (int64_t c0 = 0; c0 < m2; c0 += T2) {
+                    const int64_t n2 = std::min(T2, m2 - c0);
+                    for (int64_t c = 0; c < n2; ++c)
+                        for (int64_t r = 0; r < n1; ++r) {
+                            const int64_t k = r0 + r + tr_m1 * (c0 + c), mk_ = (m - k) & (m - 1);
+                            double* q = &buf[4 * (r * (T2 + 1) + c)];
+                            q[0] = spec[2 * k];
+                            q[1] = spec[2 * k + 1];
+                            q[2] = spec[2 * mk_];
+                            q[3] = spec[2 * mk_ + 1];
+                        }
+                    for (int64_t r = 0; r < n1; ++r)
+                        for (int64_t c = 0; c < n2; ++c) {
+                            const double* q = &buf[4 * (r * (T2 + 1) + c)];
+                            put(q, q + 2, (r0 + r) * m2 + c0 + c);
+                        }
+                }
+            }
+        } else {
+            for (int64_t k = 0; k < m; ++k) put(&spec[2 * k], &spec[2 * ((m - k) & (m - 1))], k);
         }
         if ((rc = up(bc.ch, &bc.chirp))) return rc;
         for (int d = 0; d < 2; ++d)
@@ -1107,11 +1134,10 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     const int es = prec ? 16 : 8;
     if (j.in_nd != 1 || j.out_nd != 1) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "Bluestein needs unit stride");
     const int64_t n = j.n, m = next_pow2(2 * n - 1);
-    BlueTables bt;
-    // the inverse scale rides on the post-multiply table in the chained form
-    int rc = blue_tables(p, n, m, di ? j.scale : 1.0, bt);
-    if (rc) return rc;
     if (m <= max_single_pass(prec)) {
+        BlueTables bt;
+        int rc = blue_tables(p, n, m, 1.0, bt);
+        if (rc) return rc;
         const KernelInfo* k = find_kernel(prec, (int)m, VAR_BLUE, dir);
         if (!k) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no Bluestein kernel for M=" + std::to_string(m));
         KArgs dummy{};
@@ -1149,75 +1175,73 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
         algo += "bluestein" + std::to_string(n) + "m" + std::to_string(m);
         return AFFT_OK;
     }
-    // chained form on the four-step kernels of M = m1*m2
+    // chained form of M = m1*m2: column pass (chirp and zero padding fused
+    // into its loads), row pass (k_bluemid: forward FFT, filter, inverse FFT),
+    // inverse column pass (post-chirp and crop fused into its stores), all in
+    // place in TMP0
     const int lg = ilog2(m);
-    const int64_t m1 = 1LL << (lg / 2), m2 = m / m1;
+    // Rows of 4096 points where that leaves columns of 128 to 1024 points.
+    // Complex128 1,000,003 points x 8 (M = 2^21) with m1 = 128, 256, 512, 1024:
+    // 0.403, 0.384, 0.384, 0.390 ms; complex64 40,009 x 256 (M = 2^17) with 128,
+    // 256, 512: 0.272, 0.310, 0.296.
+    int64_t m1 = std::max<int64_t>(128, m / 4096);
+    if (m1 > 1024) m1 = 1LL << (lg / 2);
+    const int64_t m2 = m / m1;
     if (m2 > max_single_pass(prec)) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "Bluestein length too large");
-    const KernelInfo* ka[2] = {find_kernel(prec, (int)m1, VAR_4A, -1), find_kernel(prec, (int)m1, VAR_4A, 1)};
-    const KernelInfo* kb[2] = {find_kernel(prec, (int)m2, VAR_4B, -1), find_kernel(prec, (int)m2, VAR_4B, 1)};
-    if (!ka[0] || !ka[1] || !kb[0] || !kb[1]) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "missing four-step kernel");
-    // chunks of transforms whose two M-point intermediates stay in the
-    // last-level cache between the four passes
-    const int64_t cc = std::min<int64_t>(j.count, std::max<int64_t>(1, (int64_t)(fourstep_chunk_bytes() / (size_t)(2 * m * es))));
+    const KernelInfo* ka = find_kernel(prec, (int)m1, VAR_4A, -1);
+    const KernelInfo* kr = find_kernel(prec, (int)m2, VAR_BLUEMID, -1);
+    const KernelInfo* kc = find_kernel(prec, (int)m1, VAR_COL, 1);
+    if (!ka || !kr || !kc) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "missing Bluestein chain kernel");
+    BlueTables bt;
+    // the inverse scale rides on the post-multiply table
+    int rc = blue_tables(p, n, m, di ? j.scale : 1.0, bt, m1);
+    if (rc) return rc;
+    // chunks of transforms whose M-point intermediate stays in the last-level
+    // cache between the three passes
+    const int64_t cc = std::min<int64_t>(j.count, std::max<int64_t>(1, (int64_t)(fourstep_chunk_bytes() / (size_t)(m * es))));
     const size_t need = (size_t)(cc * m * es);
-    for (int t = 0; t < 2; ++t)
-        if (need > p.tmp_bytes[t]) p.tmp_bytes[t] = need;
-    KArgs A[2]{}, B[2]{};
-    for (int d = 0; d < 2; ++d) {
-        if ((rc = schedule_twiddles(p, ka[d], &A[d].tw))) return rc;
-        if ((rc = schedule_twiddles(p, kb[d], &B[d].tw))) return rc;
-        if ((rc = split_twiddles(p, prec, m, &A[d].tw4_shift, &A[d].tw4_lo, &A[d].tw4_hi))) return rc;
-        A[d].tw4_L = m;
-        A[d].count = m2;
-        A[d].in_cd = 1; A[d].in_nd = m2; A[d].out_cd = 1; A[d].out_nd = m2;
-        A[d].out_bd = m;
-        A[d].scale = 1.0;
-        B[d].count = m1;
-        B[d].in_cd = m2; B[d].in_nd = 1; B[d].in_bd = m;
-        B[d].out_cd = 1; B[d].out_nd = m1;
-        B[d].scale = 1.0;
-        A[d].xcd = xcd_order(m2 * es, m2 * es);
-        B[d].xcd = xcd_order(m2 * es, m1 * es);
-    }
-    // A1: chirp-multiply + zero-pad fused into the first column pass
-    A[0].fuse = FUSE_CHIRP_IN;
-    A[0].fvec = bt.chirp;
-    A[0].fconj = di;
-    A[0].flen = n;
-    // B1: pointwise filter product fused into the transposing store
-    B[0].fuse = FUSE_MUL_OUT;
-    B[0].fvec = bt.filt[di];
-    B[0].flen = m;
-    B[0].out_bd = m;
-    // B2: post-chirp (and 1/N for the inverse), cropped to n points
-    B[1].fuse = FUSE_CROP_OUT;
-    B[1].fvec = bt.post[di];
-    B[1].flen = n;
+    if (need > p.tmp_bytes[0]) p.tmp_bytes[0] = need;
+    KArgs A{}, R{}, C{};
+    if ((rc = schedule_twiddles(p, ka, &A.tw))) return rc;
+    if ((rc = split_twiddles(p, prec, m, &A.tw4_shift, &A.tw4_lo, &A.tw4_hi))) return rc;
+    A.tw4_L = m;
+    A.count = m2;
+    A.in_cd = 1; A.in_nd = m2; A.in_bd = j.in_cd;
+    A.out_cd = 1; A.out_nd = m2; A.out_bd = m;
+    A.scale = 1.0;
+    A.xcd = xcd_order(m2 * es, m2 * es);
+    A.fuse = FUSE_CHIRP_IN;
+    A.fvec = bt.chirp;
+    A.fconj = di;
+    A.flen = n;
+    if ((rc = schedule_twiddles(p, kr, &R.tw))) return rc;
+    R.tw4_shift = A.tw4_shift; R.tw4_lo = A.tw4_lo; R.tw4_hi = A.tw4_hi; R.tw4_L = m;
+    R.count = m1;
+    R.in_cd = R.out_cd = m2; R.in_nd = R.out_nd = 1; R.in_bd = R.out_bd = m;
+    R.scale = 1.0;
+    R.fvec = bt.filt[di];
+    if ((rc = schedule_twiddles(p, kc, &C.tw))) return rc;
+    C.count = m2;
+    C.in_cd = C.out_cd = 1; C.in_nd = C.out_nd = m2; C.in_bd = m; C.out_bd = j.out_cd;
+    C.scale = 1.0;
+    C.xcd = A.xcd;
+    C.fuse = FUSE_CROP_OUT;
+    C.fvec = bt.post[di];
+    C.flen = n;
     for (int64_t y = 0; y < j.slices; ++y) {
         for (int64_t c0 = 0; c0 < j.count; c0 += cc) {
             const int64_t cnt = std::min(cc, j.count - c0);
-            KArgs a1 = A[0];
-            a1.in_bd = j.in_cd;
-            Step s1 = make_step(ka[0], a1, (m2 + ka[0]->tpb - 1) / ka[0]->tpb, 1, "blueA1");
+            Step s1 = make_step(ka, A, (m2 + ka->tpb - 1) / ka->tpb, 1, "blueA");
             s1.in_role = j.in_role; s1.in_off = j.in_off + (y * j.in_bd + c0 * j.in_cd) * es;
             s1.out_role = ROLE_TMP0; s1.out_off = 0;
             push_sliced(p.steps[di], s1, cnt, j.in_cd * es, m * es);
-            Step s2 = make_step(kb[0], B[0], (m1 + kb[0]->tpb - 1) / kb[0]->tpb, 1, "blueB1");
-            s2.in_role = ROLE_TMP0; s2.in_off = 0;
-            s2.out_role = ROLE_TMP1; s2.out_off = 0;
+            Step s2 = make_step(kr, R, (m1 + kr->tpb - 1) / kr->tpb, 1, "blueR");
+            s2.in_role = s2.out_role = ROLE_TMP0; s2.in_off = s2.out_off = 0;
             push_sliced(p.steps[di], s2, cnt, m * es, m * es);
-            KArgs a2 = A[1];
-            a2.in_bd = m;
-            Step s3 = make_step(ka[1], a2, (m2 + ka[1]->tpb - 1) / ka[1]->tpb, 1, "blueA2");
-            s3.in_role = ROLE_TMP1; s3.in_off = 0;
-            s3.out_role = ROLE_TMP0; s3.out_off = 0;
-            push_sliced(p.steps[di], s3, cnt, m * es, m * es);
-            KArgs b2 = B[1];
-            b2.out_bd = j.out_cd;
-            Step s4 = make_step(kb[1], b2, (m1 + kb[1]->tpb - 1) / kb[1]->tpb, 1, "blueB2");
-            s4.in_role = ROLE_TMP0; s4.in_off = 0;
-            s4.out_role = j.out_role; s4.out_off = j.out_off + (y * j.out_bd + c0 * j.out_cd) * es;
-            push_sliced(p.steps[di], s4, cnt, m * es, j.out_cd * es);
+            Step s3 = make_step(kc, C, (m2 + kc->tpb - 1) / kc->tpb, 1, "blueC");
+            s3.in_role = ROLE_TMP0; s3.in_off = 0;
+            s3.out_role = j.out_role; s3.out_off = j.out_off + (y * j.out_bd + c0 * j.out_cd) * es;
+            push_sliced(p.steps[di], s3, cnt, m * es, j.out_cd * es);
         }
     }
     if (!algo.empty()) algo += "+";

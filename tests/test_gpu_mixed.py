@@ -1,7 +1,8 @@
 """The composite-radix runtime kernel (kmix.hpp) where its launch shapes have
 edges: every radix alone, groups that leave a partial block, several
 butterflies a thread, prime-power and longest lengths, in place, strided
-columns, and four-step factors of a single pass; against the oracle, within
+columns, four-step factors of a single pass, real rows, and the three-pass
+Bluestein chain; against the oracle (numpy for the last), within
 the library's budgets (helpers.c64_tol, C128_TOL)."""
 import numpy as np
 import pytest
@@ -112,3 +113,19 @@ def test_real_rows_over_their_own_input(ctx, dims, noalloc):
                 got = torch.view_as_complex(buf.view(-1, 2)).cpu().numpy().reshape(X.shape)
                 assert rel_l2(got, X) <= c64_tol(x[0].size)
     assert rel_l2(buf[:x.size].cpu().numpy().reshape(x.shape), x) <= 2 * c64_tol(x[0].size)
+
+
+# three-pass Bluestein chains: padded lengths from the first beyond LDS, rows of
+# 128 to 4096 points, both directions
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n", [4099, 8209, 11 * 1009, 17 * 1031, 70001, 150001, 300007])
+def test_bluestein_chain(ctx, n, prec, dt):
+    batch = max(1, min(3, 400000 // n))
+    x = synth.uniform_complex(n, (batch, n), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch) as p:
+        got = np.empty_like(x)
+        p.forward(got, x)
+        back = got.copy()
+        p.inverse(back, back)
+    assert rel_l2(got, np.fft.fft(x.astype(np.complex128), axis=1)) <= _tol(prec, n)
+    assert rel_l2(back, np.fft.ifft(got.astype(np.complex128), axis=1)) <= _tol(prec, n)
