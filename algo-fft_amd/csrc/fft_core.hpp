@@ -162,4 +162,20 @@ __device__ __forceinline__ void core(cx<T> (&v)[E], cx<T>* lds, int t, TW tw, co
     core_all<T, S, E, DIR, HOIST>(v, lds, t, tw, li, std::make_integer_sequence<int, S::P>{});
 }
 
+// As core, with the last pass on another thread mapping: thread tl of the
+// transform that ll addresses reads its inputs from LDS and ends with points
+// tl + TT*e of it in registers.  For row blocks whose store runs across the
+// transforms.
+template <typename T, class S, int E, int DIR, class TW, class L, int... Ps>
+__device__ __forceinline__ void core_head(cx<T> (&v)[E], cx<T>* lds, int t, TW tw, const L& li,
+                                          std::integer_sequence<int, Ps...>) {
+    (core_pass<T, S, E, DIR, Ps, false>(v, lds, t, tw, li), ...);
+}
+template <typename T, class S, int E, int DIR, class TW, class L>
+__device__ __forceinline__ void core_turn(cx<T> (&v)[E], cx<T>* lds, int t, TW tw, const L& li, int tl, const L& ll) {
+    static_assert(S::P > 1, "one pass exchanges nothing");
+    core_head<T, S, E, DIR>(v, lds, t, tw, li, std::make_integer_sequence<int, S::P - 1>{});
+    core_pass<T, S, E, DIR, S::P - 1, false>(v, lds, tl, tw, ll);
+}
+
 }  // namespace afft
