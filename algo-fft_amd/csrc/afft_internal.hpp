@@ -145,6 +145,13 @@ struct MixArgs;
 // of `count` transforms of n points, n 7-smooth and at most gen_row_cap.
 int mix_row_launch(Plan& p, int64_t n, int64_t count, MixArgs& a, int* threads, int* lds);
 int prep_dynamic_lds(const void* fn, int lds);
+// Radices of n 7-smooth points on tpt threads a transform (at most 16 points a
+// thread) in LDS rows of the given pitch, every pass in place: the fewest
+// passes, then the least idle lanes and bank conflicts.
+std::vector<int> mix_lds_schedule(int64_t n, int prec, int tpt, int pitch);
+// Appends the twiddles of a pass (mix_twiddle's entries) to tw and returns it.
+struct MixPass;
+MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw);
 struct BlueTables {
     const void* chirp = nullptr;                 // n entries, forward sign
     const void* filt[2] = {nullptr, nullptr};    // [fwd, inv], m entries, 1/m folded in

@@ -59,7 +59,7 @@ struct MixCfg {
 // Twiddle entries loaded per butterfly: every power for radices up to 8, else
 // w^1, w^2, w^3 and w^4, w^8, w^12, w^16, whose products give the others (one
 // product each).  Entry i * Ns + k of the pass's table is the i-th of them for
-// butterfly k.  A radix-10 butterfly loads 5 values instead of 9: with every
+// butterfly k; tw is a const cx<T>* or a gptr<cx<T>>.  A radix-10 butterfly loads 5 values instead of 9: with every
 // power loaded complex64 rows of 960 points took 0.233 ms instead of 0.203,
 // complex128 rows of 1500 0.236 instead of 0.209.  Issuing the loads before
 // the barrier in front of the pass lost 2-8 % (registers).  Fewer loads (w^1,
@@ -68,8 +68,8 @@ struct MixCfg {
 __host__ __device__ constexpr int mix_ntw(int R) { return R <= 8 ? R - 1 : 3 + (R - 1) / 4; }
 __host__ __device__ constexpr int mix_twpow(int R, int i) { return R <= 8 || i < 3 ? i + 1 : 4 * (i - 2); }
 
-template <int R, int DIR, typename T>
-__device__ __forceinline__ void mix_twiddle(const cx<T>* __restrict__ tw, int NS, int k, cx<T>* v) {
+template <int R, int DIR, typename T, class W>
+__device__ __forceinline__ void mix_twiddle(W tw, int NS, int k, cx<T>* v) {
     constexpr int NW = mix_ntw(R);
     cx<T> w[NW];
 #pragma unroll
@@ -100,9 +100,9 @@ __device__ __forceinline__ int fast_divmod(int j, int d, unsigned m, int* rem) {
 // base + r*NS.  FIRST: no twiddles (Ns = 1).  HOLD: all of the thread's
 // butterflies are read before bar() and stored after it; otherwise one after
 // the other.  Every thread of the block calls this.
-template <int R, int DIR, bool FIRST, bool HOLD, typename T, class Load, class Store, class Bar>
-__device__ __forceinline__ void mix_pass(bool act, int t, int TPT, const MixPass& ps, const cx<T>* __restrict__ tw,
-                                         Load load, Store store, Bar bar) {
+template <int R, int DIR, bool FIRST, bool HOLD, typename T, class W, class Load, class Store, class Bar>
+__device__ __forceinline__ void mix_pass(bool act, int t, int TPT, const MixPass& ps, W tw, Load load, Store store,
+                                         Bar bar) {
     constexpr int MB = mix_mb(R);
     const int NR = ps.nr, NS = ps.ns;
     if constexpr (HOLD || MB == 1) {
@@ -116,7 +116,7 @@ __device__ __forceinline__ void mix_pass(bool act, int t, int TPT, const MixPass
                 load(v[b], j, NR);
                 if constexpr (!FIRST) {
                     k[b] = fast_mod(j, NS, ps.nsm);
-                    mix_twiddle<R, DIR, T>(tw, NS, k[b], v[b]);
+                    mix_twiddle<R, DIR>(tw, NS, k[b], v[b]);
                 }
                 dft<R, DIR, 1>(v[b]);
             }
@@ -134,7 +134,7 @@ __device__ __forceinline__ void mix_pass(bool act, int t, int TPT, const MixPass
             int k = 0;
             if constexpr (!FIRST) {
                 k = fast_mod(j, NS, ps.nsm);
-                mix_twiddle<R, DIR, T>(tw, NS, k, v);
+                mix_twiddle<R, DIR>(tw, NS, k, v);
             }
             dft<R, DIR, 1>(v);
             store(v, FIRST ? j * R : (j - k) * R + k, NS);
@@ -142,9 +142,9 @@ __device__ __forceinline__ void mix_pass(bool act, int t, int TPT, const MixPass
     }
 }
 
-template <int DIR, bool FIRST, bool HOLD, typename T, class Load, class Store, class Bar>
-__device__ __forceinline__ void mix_pass_any(bool act, int t, int TPT, const MixPass& ps,
-                                             const cx<T>* __restrict__ tw, Load load, Store store, Bar bar) {
+template <int DIR, bool FIRST, bool HOLD, typename T, class W, class Load, class Store, class Bar>
+__device__ __forceinline__ void mix_pass_any(bool act, int t, int TPT, const MixPass& ps, W tw, Load load,
+                                             Store store, Bar bar) {
 #define AFFT_MIX_CASE(RR) \
     case RR: mix_pass<RR, DIR, FIRST, HOLD, T>(act, t, TPT, ps, tw, load, store, bar); break;
     switch (ps.rad) {

@@ -27,14 +27,15 @@
 // Tasks within a launch are sorted by decreasing cost on the host (a
 // longest-processing-time queue).
 //
-// Passes run in place in one LDS buffer: each thread reads all of its
-// butterflies of the pass into registers (at most ceil(16/R) of radix R,
-// since a block holds at most 4096 points), the block passes a barrier, and
-// the outputs are written back.  Global reads and writes go through staging
+// Passes are those of kmix.hpp, in place in one LDS buffer: each thread reads
+// all of its butterflies of the pass into registers (at most 16 points a
+// thread are asked for), the block passes a barrier, and the outputs are
+// written back.  Against one radix of {2, 3, 4, 5, 7, 8, 16} per pass with
+// every twiddle loaded, the 4096-job mixed set took 0.468 -> 0.455 ms.  Global reads and writes go through staging
 // loops whose lanes run along the contiguous dimension; sub-transforms sit in
 // LDS rows of pitch L + 1 so column-wise staging is free of bank conflicts.
 #pragma once
-#include "kgen.hpp"
+#include "kmix.hpp"
 
 namespace afft {
 
@@ -42,7 +43,6 @@ constexpr int RAG_THREADS = 256;
 constexpr int RAG_PTS = 4096;       // points per block (whole job, or G*L of a task)
 constexpr int RAG_BUF = 4352;       // LDS buffer in points (G*(L+1) <= 4096 + G)
 constexpr int RAG_WHOLE = 4096;     // largest sub-transform length of a split task
-constexpr int RAG_SPASS = 12;       // passes of a schedule of length <= 16384
 
 // Largest FFT length run as one task: the whole transform in 128 KiB of LDS.
 constexpr int rag_whole_cap(int prec) { return prec ? 8192 : 16384; }
@@ -58,12 +58,9 @@ struct RagW {
 };
 
 struct RSched {
-    int npass;
-    int rad[RAG_SPASS];
-    int ns[RAG_SPASS];
-    unsigned nsm[RAG_SPASS];     // mod_magic(ns[p])
-    int twoff[RAG_SPASS];
-    const void* tw;              // per-pass twiddles W_{Ns*R}^{k*r}
+    int npass;                   // runtime passes (kmix.hpp); 0 for the compile-time cores
+    MixPass p[MIX_MAXPASS];
+    const void* tw;              // per-pass twiddles
 };
 
 enum { RT_WHOLE = 0, RT_COLS = 1, RT_ROWS = 2, RT_COLS2 = 3 };
@@ -136,24 +133,57 @@ __device__ __forceinline__ cx<T> rag_tw(const RJob& jb, long long i) {
 // the last pass hands its outputs to sink(c, k, v), which may write the
 // transform's own row.  Every thread of the block calls this; the buffer is
 // complete when it returns.  TPT is a power of two.
+// The schedule is read with vector loads (the tables are written memory to the
+// compiler): readfirstlane makes its values scalars, so that the switch over
+// the radix is a scalar branch and strides stay out of the vector registers.
+__device__ __forceinline__ MixPass rag_uniform(const MixPass& p) {
+    return MixPass{__builtin_amdgcn_readfirstlane(p.rad), __builtin_amdgcn_readfirstlane(p.ns),
+                   __builtin_amdgcn_readfirstlane(p.nr), (unsigned)__builtin_amdgcn_readfirstlane((int)p.nsm),
+                   __builtin_amdgcn_readfirstlane(p.twoff)};
+}
+
 template <typename T, int DIR, class Sink>
 __device__ __forceinline__ void rag_passes(const RSched& sc, int L, int P, int cnt, int TPT, cx<T>* buf, Sink sink) {
     const int tid = threadIdx.x;
+    TPT = __builtin_amdgcn_readfirstlane(TPT);
     const int grp = tid >> (__ffs(TPT) - 1), t = tid & (TPT - 1);
     const bool active = grp < cnt;
     cx<T>* row = buf + grp * P;
     const gptr<cx<T>> tw = as_global<cx<T>>(sc.tw);
-    for (int p = 0; p < sc.npass; ++p) {
-        auto load = [&](int n) -> cx<T> { return row[n]; };
-        auto store = [&](int k, cx<T> v) { row[k] = v; };
-        auto fin = [&](int k, cx<T> v) { sink(grp, k, v); };
-        const int R = sc.rad[p];
-        if (p == sc.npass - 1)
-            rt_pass_ip_any<DIR, T>(R, active, t, TPT, L, sc.ns[p], sc.nsm[p], tw + sc.twoff[p], load, fin);
-        else
-            rt_pass_ip_any<DIR, T>(R, active, t, TPT, L, sc.ns[p], sc.nsm[p], tw + sc.twoff[p], load, store);
+    auto load = [&](auto& v, int j, int NR) __attribute__((always_inline)) {
+        constexpr int R = sizeof(v) / sizeof(v[0]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] = row[j + r * NR];
+    };
+    auto store = [&](auto& v, int base, int NS) __attribute__((always_inline)) {
+        constexpr int R = sizeof(v) / sizeof(v[0]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) row[base + r * NS] = v[r];
+    };
+    auto fin = [&](auto& v, int base, int NS) __attribute__((always_inline)) {
+        constexpr int R = sizeof(v) / sizeof(v[0]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) sink(grp, base + r * NS, v[r]);
+    };
+    auto sync = [] { __syncthreads(); };
+    const int np = __builtin_amdgcn_readfirstlane(sc.npass) - 1;
+    const MixPass p0 = rag_uniform(sc.p[0]);
+    if (np < 0) {   // one point: a copy
+        if (active && t == 0) sink(grp, 0, row[0]);
+    } else if (np == 0) {
+        mix_pass_any<DIR, true, true, T>(active, t, TPT, p0, tw, load, fin, sync);
+    } else {
+        mix_pass_any<DIR, true, true, T>(active, t, TPT, p0, tw, load, store, sync);
         __syncthreads();
+        for (int p = 1; p < np; ++p) {
+            const MixPass ps = rag_uniform(sc.p[p]);
+            mix_pass_any<DIR, false, true, T>(active, t, TPT, ps, tw + ps.twoff, load, store, sync);
+            __syncthreads();
+        }
+        const MixPass ps = rag_uniform(sc.p[np]);
+        mix_pass_any<DIR, false, true, T>(active, t, TPT, ps, tw + ps.twoff, load, fin, sync);
     }
+    __syncthreads();
 }
 
 // Staging between global memory and LDS.  A block moves at most RAG_PTS
@@ -320,12 +350,10 @@ __device__ void rag_whole_blue(const RagArgs a, const RJob& jb, cx<T>* lds) {
 // Tasks of the generic splits: at most PTS points (G <= THREADS
 // sub-transforms of L points, G*L <= PTS) on THREADS threads, 16 points per
 // thread at most, in LDS rows of pitch L + 1.  Complex64 tasks of 8192
-// points on 512 threads held to 128 VGPRs (4 waves per SIMD, 7-12 VGPRs
-// spilled) read twice the adjacent columns per row of a 4096-point task.
-// Measured on the smooth split jobs of a 4096-job mixed set: 0.146 ms with
-// 4096-point tasks (161-164 VGPRs, 3 waves per SIMD), 0.149 ms with those
-// held to 128 VGPRs, 0.162 ms with 8192-point tasks at 165 VGPRs (one block
-// per CU), 0.131 ms with them at 128, 0.139 ms with 16384-point tasks.
+// points on 512 threads (94-104 VGPRs, 4 waves per SIMD) read twice the
+// adjacent columns per row of a 4096-point task: on earlier passes the smooth
+// split jobs of a 4096-job mixed set took 0.131 ms against 0.146, 0.139 with
+// 16384-point tasks.
 template <typename T>
 struct RagG {
     static constexpr int PTS = sizeof(T) == 4 ? 8192 : RAG_PTS;
@@ -489,8 +517,8 @@ __device__ __forceinline__ void p2_row_load(const cx<T>* __restrict__ row, int t
 }
 
 // Row task: rows r0 .. r0+G-1 of S, FFT over n2 with sign SD, output
-// X[k1 + m1*k2] (scaled 1/m for the inverse), stored through LDS so that the
-// lanes of a store run along k1.
+// X[k1 + m1*k2] (scaled 1/m for the inverse); the last pass runs with lanes
+// along k1, as the stores do.
 template <typename T, int L, int SD>
 __device__ __forceinline__ void p2_rows(const RagArgs a, const RJob& jb, const RTask& tk, cx<T>* lds) {
     using S = typename P2Sched<L>::S;
@@ -499,19 +527,13 @@ __device__ __forceinline__ void p2_rows(const RagArgs a, const RJob& jb, const R
     const int r0 = tk.first;
     cx<T> v[E];
     p2_row_load<T, L>((const cx<T>*)a.scratch + jb.scr_off + (long long)(r0 + c) * L, t, v);
-    const LdsRow<L, PADSH> li(c);
-    core<T, S, E, SD>(v, lds, t, as_global<cx<T>>(jb.s[1].tw), li);
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < E; ++e) lds[li(t + TT * e)] = v[e];
-    __syncthreads();
     const int c2 = tid % G, t2 = tid / G;
-    const LdsRow<L, PADSH> li2(c2);
+    core_turn<T, S, E, SD>(v, lds, t, as_global<cx<T>>(jb.s[1].tw), LdsRow<L, PADSH>(c), t2, LdsRow<L, PADSH>(c2));
     const T sc = SD > 0 ? T(1) / T(jb.m) : T(1);
     cx<T>* __restrict__ y = (cx<T>*)a.out + jb.out_off + r0 + c2;
     const long long m1 = jb.m1;
 #pragma unroll
-    for (int e = 0; e < E; ++e) y[m1 * (t2 + TT * e)] = scl(lds[li2(t2 + TT * e)], sc);
+    for (int e = 0; e < E; ++e) y[m1 * (t2 + TT * e)] = scl(v[e], sc);
 }
 
 // Row task of a Bluestein job: forward FFT, filter product (the filter is
@@ -656,7 +678,11 @@ __device__ __forceinline__ void p2_cols2(const RagArgs a, const RJob& jb, const 
     }
 }
 
-// The persistent loop shared by the task kernels.
+// The persistent loop shared by the task kernels.  (A block's first task by its
+// own index, and the next one asked for before the current one runs, measured
+// slower on the 4096-job mixed set, 0.456 -> 0.465 and 0.471 ms: blocks that
+// wait for a CU hold back their tasks, and tasks claimed early wait behind
+// long ones.)
 template <class Run>
 __device__ __forceinline__ void rag_queue(const RagArgs a, Run run) {
     __shared__ int s_task;
@@ -664,11 +690,11 @@ __device__ __forceinline__ void rag_queue(const RagArgs a, Run run) {
     while (true) {
         if (tid == 0) s_task = atomicAdd(a.counter, 1);
         __syncthreads();
-        const int id = s_task;
+        const int id = __builtin_amdgcn_readfirstlane(s_task);
         __syncthreads();
         if (id >= a.ntasks) break;
         const RTask tk = a.tasks[id];
-        run(a.jobs[tk.job], tk);
+        run(a.jobs[__builtin_amdgcn_readfirstlane(tk.job)], tk);
     }
 }
 

@@ -677,8 +677,54 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
     return true;
 }
 
-// Kernel arguments of a launch shape; builds the twiddle tables (the
-// powers mix_twpow of every butterfly, see mix_twiddle).
+std::vector<int> mix_lds_schedule(int64_t n, int prec, int tpt, int pitch) {
+    MixShape m, best;
+    m.tpt = tpt;
+    m.g = std::max(1, 64 / tpt);
+    m.pitch = pitch;
+    double best_cost = 1e300;
+    auto extend = [&](auto&& self, int64_t rest, int passes) -> void {
+        if (rest == 1) {
+            if ((int)m.rad.size() != passes) return;
+            double cost = 0.0;
+            for (int q : m.rad) {
+                const int64_t rounds = (n / q + tpt - 1) / tpt;
+                if (rounds > mix_mb(q)) return;
+                cost += (double)tpt * rounds * q / n;
+            }
+            cost = 0.105 * cost + 0.05 * mix_bank_excess(m, n, prec, MIX_ROWS);
+            if (cost < best_cost) {
+                best_cost = cost;
+                best.rad = m.rad;
+            }
+            return;
+        }
+        if ((int)m.rad.size() == passes) return;
+        for (int q : kMixRadices) {
+            if (rest % q) continue;
+            m.rad.push_back(q);
+            self(self, rest / q, passes);
+            m.rad.pop_back();
+        }
+    };
+    for (int passes = mix_min_passes(n, MIX_MAXPASS); passes <= MIX_MAXPASS && best.rad.empty(); ++passes)
+        extend(extend, n, passes);
+    return best.rad;
+}
+
+MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw) {
+    const MixPass ps{R, (int)ns, (int)(n / R), mod_magic((unsigned)ns), (int)(tw.size() / 2)};
+    for (int w = 0; ns > 1 && w < mix_ntw(R); ++w)
+        for (int64_t k = 0; k < ns; ++k) {
+            double re, im;
+            root_of_unity(k * mix_twpow(R, w), ns * R, &re, &im);
+            tw.push_back(re);
+            tw.push_back(im);
+        }
+    return ps;
+}
+
+// Kernel arguments of a launch shape and their twiddle tables.
 static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t slices, MixArgs& a, MixShape& m) {
     if (smooth_schedule(n).empty() || !mix_shape(n, p.desc.precision, lay, count, slices, m))
         return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule");
@@ -687,16 +733,8 @@ static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t sl
     std::vector<double> tw;
     int64_t ns = 1;
     for (int i = 0; i < a.npass; ++i) {
-        const int R = m.rad[i];
-        a.p[i] = MixPass{R, (int)ns, (int)(n / R), mod_magic((unsigned)ns), (int)(tw.size() / 2)};
-        for (int w = 0; i && w < mix_ntw(R); ++w)
-            for (int64_t k = 0; k < ns; ++k) {
-                double re, im;
-                root_of_unity(k * mix_twpow(R, w), ns * R, &re, &im);
-                tw.push_back(re);
-                tw.push_back(im);
-            }
-        ns *= R;
+        a.p[i] = mix_pass_tables(n, m.rad[i], ns, tw);
+        ns *= m.rad[i];
     }
     a.tpt = m.tpt;
     a.g = m.g;

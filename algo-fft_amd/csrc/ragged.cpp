@@ -151,63 +151,48 @@ static int ragged_order_end(afft_ragged_s& r, hipStream_t s, bool track) {
     return AFFT_OK;
 }
 
-// Radix schedule and per-pass twiddles of length m (m <= rag_whole_cap), shared
-// between jobs through `cache`.  The table is r-major (entry (r-1)*Ns + k,
-// the layout of the compile-time cores) for the power-of-two split tasks and
-// k-major (entry k*(R-1) + r-1, one base address per butterfly) for the
-// runtime passes.
+// Schedule and per-pass twiddles of length m (m <= rag_whole_cap), shared
+// between jobs through `cache`: for the power-of-two split and whole tasks
+// the table of the compile-time cores (schedule_twiddles' layout, remainder
+// radix first), else the passes of kmix.hpp for rows of pitch m + 1 on the
+// fewest threads a task gives them.
 using SchedKey = std::pair<int64_t, bool>;
-static int schedule_into(Plan& tab, int prec, int64_t m, bool rmajor, RSched& j, std::map<SchedKey, RSched>& cache) {
-    const SchedKey key{m, rmajor};
+static int schedule_into(Plan& tab, int prec, int64_t m, bool cores, RSched& j, std::map<SchedKey, RSched>& cache) {
+    const SchedKey key{m, cores};
     auto it = cache.find(key);
     if (it != cache.end()) {
         j = it->second;
         return AFFT_OK;
     }
     std::memset(&j, 0, sizeof(j));
-    if (m == 1) {
-        j.npass = 1;
-        j.rad[0] = 1;
-        j.ns[0] = 1;
-        j.nsm[0] = mod_magic(1);
-        cache[key] = j;
-        return AFFT_OK;
-    }
-    std::vector<int> rad = smooth_schedule(m);
-    if (rad.empty() || (int)rad.size() > RAG_SPASS)
-        return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule for " + std::to_string(m));
-    j.npass = (int)rad.size();
-    int64_t ns = 1;
-    int off = 0;
     std::vector<double> tw;
-    for (size_t i = 0; i < rad.size(); ++i) {
-        j.rad[i] = rad[i];
-        j.ns[i] = (int)ns;
-        j.nsm[i] = mod_magic((unsigned)ns);
-        j.twoff[i] = off;
-        if (i > 0) {
-            const int R = rad[i];
-            for (int64_t e = 0; e < ns * (R - 1); ++e) {
-                const int64_t k = rmajor ? e % ns : e / (R - 1);
-                const int r = rmajor ? (int)(e / ns) + 1 : (int)(e % (R - 1)) + 1;
+    int64_t ns = 1;
+    if (cores) {
+        for (int R : smooth_schedule(m)) {
+            for (int64_t e = 0; ns > 1 && e < ns * (R - 1); ++e) {
                 double re, im;
-                root_of_unity(k * r, ns * R, &re, &im);
+                root_of_unity(e % ns * (e / ns + 1), ns * R, &re, &im);
                 tw.push_back(re);
                 tw.push_back(im);
             }
-            off += (int)(ns * (R - 1));
+            ns *= R;
         }
-        ns *= rad[i];
+    } else if (m > 1) {
+        const std::vector<int> rad = mix_lds_schedule(m, prec, (int)std::max<int64_t>(1, next_pow2(m) / 16), (int)m + 1);
+        if (rad.empty()) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule for " + std::to_string(m));
+        for (int R : rad) {
+            j.p[j.npass++] = mix_pass_tables(m, R, ns, tw);
+            ns *= R;
+        }
     }
-    int rc;
-    if (tw.empty()) {
-        j.tw = nullptr;
-    } else if (prec == 0) {
+    int rc = AFFT_OK;
+    if (!tw.empty() && prec == 0) {
         std::vector<float> f(tw.begin(), tw.end());
-        if ((rc = upload_table(tab, f.data(), f.size() * 4, &j.tw))) return rc;
-    } else {
-        if ((rc = upload_table(tab, tw.data(), tw.size() * 8, &j.tw))) return rc;
+        rc = upload_table(tab, f.data(), f.size() * 4, &j.tw);
+    } else if (!tw.empty()) {
+        rc = upload_table(tab, tw.data(), tw.size() * 8, &j.tw);
     }
+    if (rc) return rc;
     cache[key] = j;
     return AFFT_OK;
 }
@@ -446,21 +431,11 @@ static int ragged_build(afft_ragged_s& r) {
     if (!tasks.empty())
         AFFT_HIP(hipMemcpy(r.tasks_dev, tasks.data(), tasks.size() * sizeof(RTask), hipMemcpyHostToDevice));
     AFFT_HIP(hipMalloc(&r.counter, RAG_COUNTERS * sizeof(int)));
-    // Each persistent launch gets a share of the device's resident blocks,
-    // so that the concurrent branches run side by side instead of the first
-    // one filling every CU until its queue drains.  Weights 4:5:7:3 (split
-    // runtime passes, power-of-two cores, split Bluestein, whole runtime-pass
-    // and Bluestein jobs) over the branches
-    // present, 1.7 device-fulls in all, at most one device-full per branch;
-    // a set with one branch keeps the whole device.  Shares swept on the
-    // 4096-job mixed set: 0.561-0.61 ms over the settings tried with three
-    // chains; with the current chains a fourth-chain weight of 2 to 4 gives
-    // 0.468-0.469 ms, 5 or 1.9 device-fulls 0.473 ms.
-    static constexpr int weight[RAG_BRANCHES] = {4, 5, 7, 3};
-    bool present[RAG_BRANCHES] = {};
-    for (const RagLaunch& l : r.launches) present[rag_branch(l.kind)] = true;
-    int wsum = 0;
-    for (int b = 0; b < RAG_BRANCHES; ++b) wsum += present[b] ? weight[b] : 0;
+    // Each persistent launch may fill the device: the chains' launches share it
+    // as blocks come and go.  (Caps of about 0.4 to 0.6 device-fulls per chain
+    // paid while the runtime passes were slower; now the 4096-job mixed set
+    // takes 0.438 ms without and 0.455 with them, a set of 2500 jobs up to
+    // 30000 points 0.183 and 0.201.)
     for (int inv = 0; inv < 2; ++inv)
         for (RagLaunch& l : r.launches) {
             const void* fn = rag_kernel(r.prec, l, inv ? 1 : -1);
