@@ -444,8 +444,7 @@ static int ragged_build(afft_ragged_s& r) {
             int per_cu = 0;
             AFFT_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, l.threads, 0));
             const int full = std::max(1, per_cu) * std::max(1, r.ctx->props.multiProcessorCount);
-            const double share = std::min(1.0, 1.7 * weight[rag_branch(l.kind)] / std::max(1, wsum));
-            l.grid[inv] = std::max(1, (int)(full * share));
+            l.grid[inv] = std::max(1, std::min(full, l.ntask));
         }
     AFFT_HIP(hipMalloc(&r.scratch, (size_t)std::max<int64_t>(1, r.scratch_pts) * es));
     return AFFT_OK;
