@@ -174,7 +174,9 @@ def heuristic_choice(shape, cands):
     pow2 = n & (n - 1) == 0
     smooth = synth._is_smooth7(n)
     if pow2 and n <= maxp:
-        want = (STRATEGY_STOCKHAM, 0)
+        # rows of 16 points up to 512 bytes run on the runtime-radix kernel
+        short = shape.get("stride", 1) <= 1 and n >= 16 and n * (8 if prec == COMPLEX64 else 16) <= 512
+        want = (STRATEGY_MIXED, 0) if short else (STRATEGY_STOCKHAM, 0)
     elif pow2:
         lg = int(math.log2(n))
         want = (STRATEGY_SIXSTEP, 1 << TUNED_SPLIT.get((lg, prec), lg // 2))

@@ -304,6 +304,10 @@ static int emit_single(Plan& p, int di, const AxisJob& j, std::string& algo) {
     a.scale = j.scale;
     a.xcd = var == VAR_COL && xcd_order(j.in_nd * es, j.out_nd * es);
     Step s = make_step(k, a, (count + k->tpb - 1) / k->tpb, 1, var == VAR_ROW ? "row" : "col");
+    // rows whose threads cover less than a line at a time: no streaming, which
+    // would take the partial lines to memory one by one (complex64, 512 MiB: 8
+    // points 1.62 -> 0.35 ms, 16 3.47 -> 0.45, 128 0.212 -> 0.183)
+    if (var == VAR_ROW && (int64_t)(k->n / k->e) * es < 128) s.nt_mask = 0;
     s.in_role = j.in_role;
     s.out_role = j.out_role;
     s.in_off = j.in_off;
@@ -1378,6 +1382,17 @@ static int emit_axis_direct(Plan& p, int di, const AxisJob& j, std::string& algo
     default:
         return set_error(AFFT_ERR_NOT_IMPLEMENTED, "unknown strategy");
     }
+    // Rows of 16 points up to 512 bytes: the compile-time kernel gives a row 2
+    // to 8 threads, whose stores are partial lines; the runtime-radix kernel's
+    // go line by line.  512 MiB batches, both without streaming stores:
+    // complex64 16 points 0.449 -> 0.209 ms, 32 0.237 -> 0.206, 64 0.203 ->
+    // 0.184; complex128 16 0.304 -> 0.177, 32 0.198 -> 0.172.  8 points and
+    // fewer are one thread's either way (complex64 8 points 0.350 against
+    // 0.388), and at 1 KiB the compile-time kernel wins on cached batches
+    // (complex64 128 points, 32 MiB: 11.7 against 14.2 us).
+    if (is_pow2(j.n) && rows && j.n >= 16 && j.n * (prec ? 16 : 8) <= 512 &&
+        !(p.desc.flags & AFFT_FLAG_MFMA))
+        return emit_gen_single(p, di, j, algo);
     if (is_pow2(j.n) && j.n <= max_single_pass(prec)) return emit_single(p, di, j, algo);
     if (is_pow2(j.n)) return emit_fourstep(p, di, j, algo);
     if (!smooth_schedule(j.n).empty()) {

@@ -129,3 +129,23 @@ def test_bluestein_chain(ctx, n, prec, dt):
         p.inverse(back, back)
     assert rel_l2(got, np.fft.fft(x.astype(np.complex128), axis=1)) <= _tol(prec, n)
     assert rel_l2(back, np.fft.ifft(got.astype(np.complex128), axis=1)) <= _tol(prec, n)
+
+
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64, 128])
+@pytest.mark.parametrize("batch", [1, 67, 4099])
+def test_short_power_of_two_rows(ctx, n, batch, prec, dt):
+    # 16 points up to 512 bytes are this kernel's, the others the compile-time
+    # kernel's; a forced strategy keeps the latter at every length
+    x = synth.uniform_complex(11 * n + batch, (batch, n), dt)
+    short = 16 <= n <= (64 if prec == A.COMPLEX64 else 32)
+    ref = O.fft_batch(x.astype(np.complex128))
+    for strategy in (A.STRATEGY_AUTO, A.STRATEGY_STOCKHAM):
+        with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch, strategy=strategy) as p:
+            assert p.describe().startswith("hip_mixed") == (short and strategy == A.STRATEGY_AUTO)
+            got = np.empty_like(x)
+            p.forward(got, x)
+            back = got.copy()
+            p.inverse(back, back)   # in place
+        assert rel_l2(got, ref) <= _tol(prec, n)
+        assert rel_l2(back, O.fft_batch(got.astype(np.complex128), inverse=True)) <= _tol(prec, n)
