@@ -94,6 +94,7 @@ struct BlueCache {
     std::vector<double> ch;
     const void* chirp = nullptr;
     const void* filt[2] = {nullptr, nullptr};
+    const void* perm = nullptr;
 };
 
 struct Plan {
@@ -156,8 +157,12 @@ struct BlueTables {
     const void* chirp = nullptr;                 // n entries, forward sign
     const void* filt[2] = {nullptr, nullptr};    // [fwd, inv], m entries, 1/m folded in
     const void* post[2] = {nullptr, nullptr};    // [fwd, inv]: chirp, conj(chirp)*inv_scale
+    const void* perm = nullptr;                  // Rader: g^q mod n, uint16
 };
 // tr_m1 > 0 stores the filter spectra row-major as [k1][k2], k = k1 + tr_m1*k2
+// (m a power of two); BLUE_RADER: filter and permutation of a prime n,
+// m = n - 1, no chirp
+constexpr int64_t BLUE_RADER = -1;
 int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt, int64_t tr_m1 = 0);
 // W_L^i = hi[i >> shift] * lo[i & (2^shift - 1)], both FP64-generated
 int split_twiddles(Plan& p, int prec, int64_t L, int* shift, const void** lo, const void** hi);

@@ -14,9 +14,10 @@
 #include <cstring>
 
 #include <cmath>
+#include <complex>
 
 #include "afft_internal.hpp"
-#include "kmix.hpp"
+#include "kblue.hpp"
 
 namespace afft {
 
@@ -598,7 +599,9 @@ static int mix_min_passes(int64_t n, int most) {
 // times the group sizes; the bank conflicts rank the cheapest of them.
 // Radices up to 10 hold 16 points per thread, so at most n/16 threads (the
 // largest block at the largest length) always fit.
-static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out) {
+// pad: LDS slots of a row beyond its n points.
+static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out,
+                      double* cost = nullptr, int pad = 0) {
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
     const double conf = lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012;
     const int minp = mix_min_passes(n, MIX_MAXPASS);
@@ -633,7 +636,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
                 if (m.g == last_g) continue;
                 last_g = m.g;
                 if (m.g > 1 && m.g >= 2 * count) continue;
-                m.pitch = (int)(lay == MIX_TROWS ? n | 1 : n);
+                m.pitch = (int)(lay == MIX_TROWS ? n | 1 : n + pad);
                 const int64_t lds = (int64_t)m.g * m.pitch * es;
                 if ((int64_t)m.g * m.tpt > maxth || lds > 163840) continue;
                 m.lds = (int)lds;
@@ -678,6 +681,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
             out = t.second;
         }
     }
+    if (cost) *cost = best;
     return true;
 }
 
@@ -729,8 +733,9 @@ MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw) {
 }
 
 // Kernel arguments of a launch shape and their twiddle tables.
-static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t slices, MixArgs& a, MixShape& m) {
-    if (smooth_schedule(n).empty() || !mix_shape(n, p.desc.precision, lay, count, slices, m))
+static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t slices, MixArgs& a, MixShape& m,
+                    int pad = 0) {
+    if (smooth_schedule(n).empty() || !mix_shape(n, p.desc.precision, lay, count, slices, m, nullptr, pad))
         return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no radix schedule");
     a.n = (int)n;
     a.npass = (int)m.rad.size();
@@ -1004,9 +1009,33 @@ static void host_fft_ld(std::vector<long double>& re, std::vector<long double>& 
     }
 }
 
-// Forward spectrum of one sequence of m = 2^k complex128 points (interleaved
-// re, im in `v`, replaced by its DFT), on the plan's device with a complex128
-// plan of that length forced onto the power-of-two routes (never Bluestein).
+// As host_fft_ld for any m (a product of small primes): recursive
+// decimation in time by the smallest prime factor.
+static void host_dft_ld(const std::complex<long double>* x, int64_t stride, std::complex<long double>* y, int64_t m,
+                        const std::complex<long double>* w, int64_t wstep, int64_t total) {
+    if (m == 1) {
+        y[0] = x[0];
+        return;
+    }
+    int64_t q = 2;
+    while (m % q) ++q;
+    const int64_t k1 = m / q;
+    for (int64_t r = 0; r < q; ++r) host_dft_ld(x + r * stride, stride * q, y + r * k1, k1, w, wstep * q, total);
+    std::vector<std::complex<long double>> t(q);
+    for (int64_t k = 0; k < k1; ++k) {
+        for (int64_t r = 0; r < q; ++r) t[r] = y[r * k1 + k];
+        for (int64_t s = 0; s < q; ++s) {
+            std::complex<long double> a = t[0];
+            for (int64_t r = 1; r < q; ++r) a += t[r] * w[(r * (k + s * k1) % m) * wstep % total];
+            y[s * k1 + k] = a;
+        }
+    }
+}
+
+// Forward spectrum of one sequence of m complex128 points, m 7-smooth
+// (interleaved re, im in `v`, replaced by its DFT), on the plan's device with a
+// complex128 plan of that length, powers of two forced onto their routes
+// (never Bluestein).
 static int device_fft_c128(Plan& p, std::vector<double>& v, int64_t m) {
     afft_plan_desc d{};
     d.kind = AFFT_C2C;
@@ -1014,7 +1043,9 @@ static int device_fft_c128(Plan& p, std::vector<double>& v, int64_t m) {
     d.rank = 1;
     d.dims[0] = m;
     d.batch = 1;
-    d.strategy = m <= max_single_pass(1) ? AFFT_STRATEGY_STOCKHAM : AFFT_STRATEGY_SIXSTEP;
+    d.strategy = m > (is_pow2(m) ? max_single_pass(1) : gen_row_cap(1)) ? AFFT_STRATEGY_SIXSTEP
+                 : is_pow2(m)                                           ? AFFT_STRATEGY_STOCKHAM
+                                                                        : AFFT_STRATEGY_MIXED;
     afft_plan sub = nullptr;
     int rc = afft_plan_create_desc(static_cast<afft_context>(p.ctx), &d, &sub);
     if (rc) return rc;
@@ -1068,6 +1099,32 @@ static void bluestein_chirp(int64_t n, bool refchirp, std::vector<double>& ch) {
     }
 }
 
+// A generator of the multiplicative group modulo a prime n.
+static int64_t primitive_root(int64_t n) {
+    std::vector<int64_t> f;
+    for (int64_t r = n - 1, q = 2; r > 1; ++q)
+        if (r % q == 0) {
+            f.push_back(q);
+            while (r % q == 0) r /= q;
+        }
+    for (int64_t g = 2;; ++g) {
+        bool ok = true;
+        for (int64_t q : f) {
+            int64_t x = 1, b = g;
+            for (int64_t e = (n - 1) / q; e; e >>= 1, b = b * b % n)
+                if (e & 1) x = x * b % n;
+            ok &= x != 1;
+        }
+        if (ok) return g;
+    }
+}
+
+static bool is_prime(int64_t n) {
+    for (int64_t q = 2; q * q <= n; ++q)
+        if (n % q == 0) return false;
+    return n > 1;
+}
+
 int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt, int64_t tr_m1) {
     const bool refchirp = p.desc.flags & AFFT_FLAG_REF_CHIRP;
     int rc;
@@ -1083,20 +1140,45 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
     auto it = p.blue_cache.find(key);
     if (it == p.blue_cache.end()) {
         BlueCache bc;
-        bluestein_chirp(n, refchirp, bc.ch);
+        std::vector<double> spec(2 * m, 0.0);
+        if (tr_m1 == BLUE_RADER) {
+            // b[q] = W_n^(g^-q), q < m = n - 1
+            std::vector<unsigned short> perm(m);
+            const int64_t gen = primitive_root(n);
+            for (int64_t q = 0, x = 1; q < m; x = x * gen % n, ++q) {
+                perm[q] = (unsigned short)x;
+                const int64_t at = q ? m - q : 0;
+                root_of_unity(x, n, &spec[2 * at], &spec[2 * at + 1]);
+            }
+            if ((rc = upload_table(p, perm.data(), perm.size() * 2, &bc.perm))) return rc;
+        } else {
+            bluestein_chirp(n, refchirp, bc.ch);
         // Forward filter b[k] = conj(chirp[k]), mirrored (b[m-k] = b[k]), zero
         // between.  Its spectrum B: a long-double host FFT up to 4096 points,
         // above that one complex128 FFT on the device (each costs about
         // 0.1-0.5 ms around 4096 points).  The inverse filter is
         // conj(b), whose spectrum is conj(B[-k mod m]).
-        std::vector<double> spec(2 * m, 0.0);
-        spec[0] = bc.ch[0];
-        spec[1] = -bc.ch[1];
-        for (int64_t k = 1; k < n; ++k) {
-            spec[2 * k] = spec[2 * (m - k)] = bc.ch[2 * k];
-            spec[2 * k + 1] = spec[2 * (m - k) + 1] = -bc.ch[2 * k + 1];
+            spec[0] = bc.ch[0];
+            spec[1] = -bc.ch[1];
+            for (int64_t k = 1; k < n; ++k) {
+                spec[2 * k] = spec[2 * (m - k)] = bc.ch[2 * k];
+                spec[2 * k + 1] = spec[2 * (m - k) + 1] = -bc.ch[2 * k + 1];
+            }
         }
-        if (m <= 4096) {
+        if (m <= 4096 && !is_pow2(m)) {
+            std::vector<std::complex<long double>> x(m), y(m), w(m);
+            for (int64_t k = 0; k < m; ++k) {
+                x[k] = {spec[2 * k], spec[2 * k + 1]};
+                long double re, im;
+                root_of_unity_ld(k, m, &re, &im);
+                w[k] = {re, im};
+            }
+            host_dft_ld(x.data(), 1, y.data(), m, w.data(), 1, m);
+            for (int64_t k = 0; k < m; ++k) {
+                spec[2 * k] = (double)y[k].real();
+                spec[2 * k + 1] = (double)y[k].imag();
+            }
+        } else if (m <= 4096) {
             std::vector<long double> re(m), im(m);
             for (int64_t k = 0; k < m; ++k) {
                 re[k] = spec[2 * k];
@@ -1113,16 +1195,18 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
         std::vector<double> filt[2];
         // natural order, or row-major [k1][k2] of k = k1 + tr_m1 * k2
         const int64_t m2 = tr_m1 > 0 ? m / tr_m1 : 0;
-        const double inv_m = 1.0 / (double)m;   // m is a power of two: exact
+        const double dm = (double)m, inv_m = 1.0 / dm;
+        const bool exact = is_pow2(m);   // then x * inv_m == x / m, and far cheaper
+        auto div = [&](double x) { return exact ? x * inv_m : x / dm; };
         for (int d = 0; d < 2; ++d) filt[d].resize(2 * m);
         // filt[0][at] = spec[k] / m, filt[1][at] = conj(spec[-k mod m]) / m,
         // through a buffer where the order changes (runs of 32 points read,
         // of 256 points written)
         auto put = [&](const double* f, const double* r, int64_t at) {
-            filt[0][2 * at] = f[0] * inv_m;
-            filt[0][2 * at + 1] = f[1] * inv_m;
-            filt[1][2 * at] = r[0] * inv_m;
-            filt[1][2 * at + 1] = -r[1] * inv_m;
+            filt[0][2 * at] = div(f[0]);
+            filt[0][2 * at + 1] = div(f[1]);
+            filt[1][2 * at] = div(r[0]);
+            filt[1][2 * at + 1] = div(-r[1]);
         };
         if (tr_m1 > 0) {
             constexpr int64_t T1 = 32, T2 = 256;
@@ -1133,7 +1217,7 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
                     const int64_t n2 = std::min(T2, m2 - c0);
                     for (int64_t c = 0; c < n2; ++c)
                         for (int64_t r = 0; r < n1; ++r) {
-                            const int64_t k = r0 + r + tr_m1 * (c0 + c), mk_ = (m - k) & (m - 1);
+                            const int64_t k = r0 + r + tr_m1 * (c0 + c), mk_ = (m - k) & (m - 1);   // m is a power of two here
                             double* q = &buf[4 * (r * (T2 + 1) + c)];
                             q[0] = spec[2 * k];
                             q[1] = spec[2 * k + 1];
@@ -1148,9 +1232,9 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
                 }
             }
         } else {
-            for (int64_t k = 0; k < m; ++k) put(&spec[2 * k], &spec[2 * ((m - k) & (m - 1))], k);
+            for (int64_t k = 0; k < m; ++k) put(&spec[2 * k], &spec[k ? 2 * (m - k) : 0], k);
         }
-        if ((rc = up(bc.ch, &bc.chirp))) return rc;
+        if (tr_m1 != BLUE_RADER && (rc = up(bc.ch, &bc.chirp))) return rc;
         for (int d = 0; d < 2; ++d)
             if ((rc = up(filt[d], &bc.filt[d]))) return rc;
         it = p.blue_cache.emplace(key, std::move(bc)).first;
@@ -1159,6 +1243,8 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
     bt.chirp = it->second.chirp;
     bt.filt[0] = it->second.filt[0];
     bt.filt[1] = it->second.filt[1];
+    bt.perm = it->second.perm;
+    if (tr_m1 == BLUE_RADER) return AFFT_OK;
     // post-multiply tables: the chirp itself (forward), conj(chirp) times the
     // inverse scale (inverse)
     bt.post[0] = bt.chirp;
@@ -1170,12 +1256,112 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
     return up(post, &bt.post[1]);
 }
 
+const void* mix_blue_kernel_c64();
+const void* mix_blue_kernel_c128();
+const void* mix_rader_kernel_c64();
+const void* mix_rader_kernel_c128();
+
+// Rows of a length with a prime factor above 7 on k_mix_blue (kblue.hpp):
+// Rader's form (m = n - 1) or Bluestein's with a 7-smooth m >= 2n - 1.
+static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rader, std::string& algo) {
+    const int prec = p.desc.precision;
+    const int es = prec ? 16 : 8;
+    BlueTables bt;
+    MixBlueArgs a{};
+    MixShape ms;
+    int rc = blue_tables(p, j.n, m, 1.0, bt, rader ? BLUE_RADER : 0);
+    if (rc || (rc = mix_args(p, m, MIX_ROWS, j.count, j.slices, a.m, ms, rader ? 1 : 0))) return rc;
+    const void* fn = rader ? (prec ? mix_rader_kernel_c128() : mix_rader_kernel_c64())
+                           : (prec ? mix_blue_kernel_c128() : mix_blue_kernel_c64());
+    if ((rc = prep_dynamic_lds(fn, ms.lds))) return rc;
+    a.chirp = bt.chirp;
+    a.filt = bt.filt[di];
+    a.perm = (const unsigned short*)bt.perm;
+    a.n = (int)j.n;
+    a.inverse = di;
+    a.m.k.count = j.count;
+    a.m.k.in_cd = j.in_cd;
+    a.m.k.out_cd = j.out_cd;
+    a.m.k.scale = j.scale;
+    const std::string name = (rader ? "rader" : "bluestein") + std::to_string(j.n);
+    for (int64_t y = 0; y < j.slices; ++y) {
+        Step s;
+        s.fn = fn;
+        s.grid = dim3((unsigned)((j.count + ms.g - 1) / ms.g), 1, 1);
+        s.block = dim3((unsigned)ms.threads, 1, 1);
+        s.lds_bytes = ms.lds;
+        s.arg.resize(sizeof(MixBlueArgs));
+        std::memcpy(s.arg.data(), &a, sizeof(MixBlueArgs));
+        s.in_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, in));
+        s.out_field = (int)(offsetof(MixArgs, k) + offsetof(KArgs, out));
+        s.in_role = j.in_role;
+        s.out_role = j.out_role;
+        s.in_off = j.in_off + y * j.in_bd * es;
+        s.out_off = j.out_off + y * j.out_bd * es;
+        s.name = name;
+        p.steps[di].push_back(s);
+    }
+    if (!algo.empty()) algo += "+";
+    algo += name + (rader ? "" : "m" + std::to_string(m));
+    return AFFT_OK;
+}
+
+// The 7-smooth M >= 2n - 1 that k_mix_blue should take for n, 0 where the power
+// of two m does better.  Among the first eight that fit in LDS the least
+// modelled time: the launch shape's cost, in which both transforms share the
+// trip through memory (0.98 to 1.24 of the best of nine measured at 27 lengths
+// from 22 to 9797, mean 1.02).
+//
+// A point of the compile-time kernel (k_blue) costs less, so M has to be
+// shorter by a factor.  2^24 complex64 points, power of two -> M: 131 points 512
+// 0.185 ms -> 270 0.109; 341 1024 0.150 -> 686 0.134; 611 2048 0.143 -> 1260
+// 0.148; 1111 4096 0.164 -> 2268 0.150; 1313 4096 0.146 -> 2700 0.155; 2053 8192 0.354
+// -> 4200 0.191; 6001 16384 0.266 -> 12096 0.215.  2^23 complex128 points: 143 512 0.152
+// -> 288 0.114; 703 2048 0.135 -> 1440 0.124; 1529 4096 0.135 -> 3072 0.134; 2587 8192
+// 0.217 -> 5184 0.243.  Against the three-pass chain always: complex64 8209
+// points 0.511 -> 0.239 ms, complex128 4099 0.530 -> 0.233.
+static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count, int64_t slices) {
+    double factor = 1.0;
+    if (m < 256) return 0;
+    if (m <= max_single_pass(prec)) {
+        if (prec) factor = m <= 4096 ? 1.4 : 1.65;
+        else factor = m <= 1024 ? 1.45 : m <= 4096 ? 1.65 : 1.33;
+    }
+    int64_t best = 0;
+    double least = 1e300;
+    const int64_t top = std::min<int64_t>((int64_t)((double)m / factor), 163840 / (prec ? 16 : 8));
+    for (int64_t c = 2 * n - 1, seen = 0; c <= top && seen < 8; ++c) {
+        MixShape ms;
+        double cost;
+        if (smooth_schedule(c).empty() || !mix_shape(c, prec, MIX_ROWS, count, slices, ms, &cost)) continue;
+        ++seen;
+        if ((cost - 1) * (double)c < least) {
+            least = (cost - 1) * (double)c;
+            best = c;
+        }
+    }
+    return best;
+}
+
 static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) {
     const int prec = p.desc.precision;
     const int dir = di ? 1 : -1;
     const int es = prec ? 16 : 8;
     if (j.in_nd != 1 || j.out_nd != 1) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "Bluestein needs unit stride");
     const int64_t n = j.n, m = next_pow2(2 * n - 1);
+    // Plans with the reference's chirp stay on its padded lengths.  Rader's form
+    // halves the points of the convolution: primes of 2^24 complex64 points, from
+    // the padded form: 31 points 0.112 -> 0.106 ms, 257 0.215 -> 0.095, 1009 0.138
+    // -> 0.091, 4051 0.24 -> 0.126, 8101 0.22 -> 0.144; 2^23 complex128: 61 0.115 -> 0.085,
+    // 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.
+    if (!(p.desc.flags & AFFT_FLAG_REF_CHIRP)) {
+        MixShape ms;
+        if (p.desc.strategy != AFFT_STRATEGY_BLUESTEIN && n < 65536 && is_prime(n) && !smooth_schedule(n - 1).empty() &&
+            mix_shape(n - 1, prec, MIX_ROWS, j.count, j.slices, ms, nullptr, 1))
+            return emit_mix_blue(p, di, j, n - 1, true, algo);
+        if (const int64_t sm = blue_smooth_length(n, m, prec, j.count, j.slices))
+            return emit_mix_blue(p, di, j, sm, false, algo);
+    }
     if (m <= max_single_pass(prec)) {
         BlueTables bt;
         int rc = blue_tables(p, n, m, 1.0, bt);

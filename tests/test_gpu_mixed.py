@@ -149,3 +149,53 @@ def test_short_power_of_two_rows(ctx, n, batch, prec, dt):
             p.inverse(back, back)   # in place
         assert rel_l2(got, ref) <= _tol(prec, n)
         assert rel_l2(back, O.fft_batch(got.astype(np.complex128), inverse=True)) <= _tol(prec, n)
+
+
+# one-launch convolution forms of lengths with a prime factor above 7: Rader
+# (n - 1 of one to four passes, the longest of either precision) and Bluestein
+# with a padded length that is not a power of two; rows apart from each other,
+# in place, partial groups, against a forced power-of-two-or-smooth Bluestein
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n", [11, 13, 17, 19, 31, 71, 127, 257, 1009, 1459, 2017, 4051, 8101, 8641, 10369, 12289, 18433, 20161])
+@pytest.mark.parametrize("gap", [0, 3])
+def test_prime_rows(ctx, n, gap, prec, dt):
+    if (n - 1) * (16 if prec else 8) > 163840:
+        pytest.skip("longer rows take the three-pass chain")
+    batch = 67 if n < 1000 else 3
+    buf = synth.uniform_complex(n + gap, (batch, n + gap), dt)
+    x = np.ascontiguousarray(buf[:, :n])
+    ref = np.fft.fft(x.astype(np.complex128), axis=1)
+    for strategy in (A.STRATEGY_AUTO, A.STRATEGY_BLUESTEIN):
+        with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch, idist=n + gap, odist=n + gap,
+                              strategy=strategy) as p:
+            if strategy == A.STRATEGY_BLUESTEIN:
+                assert p.describe().startswith(f"hip_bluestein{n}m")
+            elif n - 1 <= (8192 if prec else 16384):
+                assert p.describe() == f"hip_rader{n}"
+            dx = torch.from_numpy(buf).cuda()
+            dy = torch.full_like(dx, 7)
+            s = torch.cuda.Stream()
+            s.wait_stream(torch.cuda.current_stream())
+            p.exec_device(A.FORWARD, dy.data_ptr(), dx.data_ptr(), s.cuda_stream)
+            s.synchronize()
+            got = dy.cpu().numpy()
+            p.exec_device(A.INVERSE, dy.data_ptr(), dy.data_ptr(), s.cuda_stream)   # in place
+            s.synchronize()
+            back = dy.cpu().numpy()
+        assert np.all(got[:, n:] == 7) and np.all(back[:, n:] == 7)
+        assert rel_l2(got[:, :n], ref) <= _tol(prec, n)
+        assert rel_l2(back[:, :n], np.fft.ifft(got[:, :n].astype(np.complex128), axis=1)) <= _tol(prec, n)
+
+
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("n", [22, 67, 69, 143, 341, 503, 703, 1111, 2053, 2587, 5117, 6002, 8209, 9797, 10201])
+def test_bluestein_rows_padded_to_smooth_lengths(ctx, n, prec, dt):
+    batch = 67 if n < 1000 else 3
+    x = synth.uniform_complex(n, (batch, n), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch) as p:
+        got = np.empty_like(x)
+        p.forward(got, x)
+        back = got.copy()
+        p.inverse(back, back)
+    assert rel_l2(got, np.fft.fft(x.astype(np.complex128), axis=1)) <= _tol(prec, n)
+    assert rel_l2(back, np.fft.ifft(got.astype(np.complex128), axis=1)) <= _tol(prec, n)
