@@ -1,4 +1,4 @@
-"""The one-launch convolution (kconv.hpp) over batches: its shortest and
+"""The one-launch convolutions (kconv.hpp, kshort.hpp) over batches: shortest and
 longest padded lengths, the first beyond them (the launches of their own),
 partial groups, odd and one-element rows, and an output over an input;
 against FP64 FFT convolution, within the library's budgets."""
@@ -78,3 +78,25 @@ def test_output_over_an_input(ctx, mode, over):
     wide = np.float64 if mode == A.CONV_REAL else np.complex128
     got = buf.cpu().numpy().reshape(batch, na + nb - 1)
     assert rel_l2(got, _ref(a.astype(wide), b.astype(wide), mode)) <= c64_tol(na + nb)
+
+
+# the direct form (kshort.hpp): its longest taps and one more, on either side,
+# tiles of 2304 (real) and 1792 (complex) outputs filled exactly, one over and
+# one under, rows of every remainder of a thread's outputs, one tap
+DIRECT = [(1, 1, 7), (5, 1, 300), (1, 5, 3), (13, 3, 100), (20, 7, 61), (40, 40, 9), (48, 48, 5), (49, 49, 5),
+          (2209, 96, 3), (2210, 96, 3), (2208, 97, 2), (1745, 48, 3), (1746, 48, 2), (48, 1744, 2), (96, 5000, 2),
+          (30000, 128, 1), (128, 40001, 1), (30000, 129, 1)]
+
+
+@pytest.mark.parametrize("na,nb,batch", DIRECT)
+@pytest.mark.parametrize("mode", [A.CONV_LINEAR, A.CONV_CORRELATE, A.CONV_REAL])
+@pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
+def test_short_sides(ctx, na, nb, batch, mode, prec):
+    a, b = _data(prec, mode, na, nb, batch)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    out = torch.full((batch * (na + nb - 1) + 5,), 7, dtype=ta.dtype, device="cuda")
+    _run(ctx, prec, mode, na, nb, batch, out, ta, tb)
+    got = out.cpu().numpy()
+    tol = c64_tol(na + nb) if prec == A.COMPLEX64 else C128_TOL
+    assert np.all(got[-5:] == 7)
+    assert rel_l2(got[:-5].reshape(batch, -1), _ref(a, b, mode)) <= tol
