@@ -1687,7 +1687,13 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
         rc = upload_table(p, w.data(), w.size() * 8, &wk);
     }
     if (rc) return rc;
-    const KernelInfo* k = (h >= 2 && is_pow2(h)) ? find_kernel(prec, (int)h, VAR_REAL, dir) : nullptr;
+    // Rows of 32 and 64 reals: as the complex ones, too few threads a row in the
+    // compile-time kernel.  256 MiB of reals, compile-time -> runtime-radix
+    // kernel, R2C / C2R: float32 32 points 0.196 / 0.179 -> 0.153 / 0.131 ms, 64 0.180 /
+    // 0.148 -> 0.150 / 0.137; float64 32 0.175 / 0.212 -> 0.120 / 0.118.  128 points
+    // are mixed (R2C 0.140 -> 0.121, C2R 0.117 -> 0.133), 16 lose (0.158 -> 0.232).
+    const bool shortr = h == 16 || h == 32;
+    const KernelInfo* k = (h >= 2 && is_pow2(h) && !shortr) ? find_kernel(prec, (int)h, VAR_REAL, dir) : nullptr;
     if (k) {
         RArgs a{};
         KArgs tmpk{};
@@ -1719,7 +1725,7 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
         return AFFT_OK;
     }
     // smooth h held in LDS: the runtime-radix kernel with the recombination
-    if (h >= 2 && !is_pow2(h) && !smooth_schedule(h).empty() && h <= gen_row_cap(prec)) {
+    if (h >= 2 && (!is_pow2(h) || shortr) && !smooth_schedule(h).empty() && h <= gen_row_cap(prec)) {
         MixRealArgs a{};
         MixShape m;
         if ((rc = mix_args(p, h, MIX_ROWS, rows, slices, a.m, m))) return rc;

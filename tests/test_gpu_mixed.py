@@ -199,3 +199,19 @@ def test_bluestein_rows_padded_to_smooth_lengths(ctx, n, prec, dt):
         p.inverse(back, back)
     assert rel_l2(got, np.fft.fft(x.astype(np.complex128), axis=1)) <= _tol(prec, n)
     assert rel_l2(back, np.fft.ifft(got.astype(np.complex128), axis=1)) <= _tol(prec, n)
+
+
+# real rows of 32 and 64 points are this kernel's, their neighbours k_real's
+@pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
+@pytest.mark.parametrize("n", [16, 32, 64, 128])
+@pytest.mark.parametrize("batch", [1, 67, 4099])
+def test_short_power_of_two_real_rows(ctx, n, batch, prec):
+    rdt, cdt = (np.float32, np.complex64) if prec == A.COMPLEX64 else (np.float64, np.complex128)
+    x = synth.uniform_real(n + batch, (batch, n), rdt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, kind=A.R2C, batch=batch) as p:
+        X = np.empty((batch, n // 2 + 1), cdt)
+        p.forward(X, x)
+        y = np.empty_like(x)
+        p.inverse(y, X)
+    assert rel_l2(X, O.rfft(x.astype(np.float64))) <= _tol(prec, n)
+    assert rel_l2(y, O.irfft(X.astype(np.complex128), n)) <= _tol(prec, n)
