@@ -1318,8 +1318,10 @@ static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rade
 // 0.148; 1111 4096 0.164 -> 2268 0.150; 1313 4096 0.146 -> 2700 0.155; 2053 8192 0.354
 // -> 4200 0.191; 6001 16384 0.266 -> 12096 0.215.  2^23 complex128 points: 143 512 0.152
 // -> 288 0.114; 703 2048 0.135 -> 1440 0.124; 1529 4096 0.135 -> 3072 0.134; 2587 8192
-// 0.217 -> 5184 0.243.  Against the three-pass chain always: complex64 8209
-// points 0.511 -> 0.239 ms, complex128 4099 0.530 -> 0.233.
+// 0.217 -> 5184 0.243.  Against the three-pass chain always, in up
+// to four passes (complex64 8209 points 0.511 -> 0.239 ms, complex128 4099 0.530
+// -> 0.233), in more with rows enough: complex64 10007 on 20480 points in six
+// passes, 64 rows 0.041 -> 0.046, 256 0.068 -> 0.050.
 static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count, int64_t slices) {
     double factor = 1.0;
     if (m < 256) return 0;
@@ -1335,6 +1337,7 @@ static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count,
         double cost;
         if (smooth_schedule(c).empty() || !mix_shape(c, prec, MIX_ROWS, count, slices, ms, &cost)) continue;
         ++seen;
+        if (m > max_single_pass(prec) && ms.rad.size() > 4 && count * slices < 256) continue;
         if ((cost - 1) * (double)c < least) {
             least = (cost - 1) * (double)c;
             best = c;
@@ -1354,7 +1357,11 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     // the padded form: 31 points 0.112 -> 0.106 ms, 257 0.215 -> 0.095, 1009 0.138
     // -> 0.091, 4051 0.24 -> 0.126, 8101 0.22 -> 0.144; 2^23 complex128: 61 0.115 -> 0.085,
     // 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.
-    if (!(p.desc.flags & AFFT_FLAG_REF_CHIRP)) {
+    // Where the power of two is beyond LDS a row is one block's, the chain spreads
+    // it over many: one launch from 64 rows on (complex128 4099 points, chain -> one
+    // launch: 1 row 19.5 -> 25.7 us, 32 27.5 -> 26.3, 64 31.3 -> 26.7, 256 67 -> 33;
+    // complex64 18433: 1 row 19.9 -> 41.5, 64 43.4 -> 42.8, 256 122 -> 52).
+    if (!(p.desc.flags & AFFT_FLAG_REF_CHIRP) && (m <= max_single_pass(prec) || j.count * j.slices >= 64)) {
         MixShape ms;
         if (p.desc.strategy != AFFT_STRATEGY_BLUESTEIN && n < 65536 && is_prime(n) && !smooth_schedule(n - 1).empty() &&
             mix_shape(n - 1, prec, MIX_ROWS, j.count, j.slices, ms, nullptr, 1))
