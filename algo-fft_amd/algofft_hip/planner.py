@@ -176,7 +176,11 @@ def heuristic_choice(shape, cands):
     if pow2 and n <= maxp:
         # rows of 16 points up to 512 bytes run on the runtime-radix kernel
         short = shape.get("stride", 1) <= 1 and n >= 16 and n * (8 if prec == COMPLEX64 else 16) <= 512
-        want = (STRATEGY_MIXED, 0) if short else (STRATEGY_STOCKHAM, 0)
+        # and so do 128 or more columns of 32 KiB to gcap points
+        es, stride, cols = (8 if prec == COMPLEX64 else 16), shape.get("stride", 1), shape.get("batch", 1)
+        many = (1 < stride and 128 <= cols <= stride and 32768 <= n * es and n <= gcap and
+                (stride * es % 8192 or stride * es * n < 256 << 20))
+        want = (STRATEGY_MIXED, 0) if short or many else (STRATEGY_STOCKHAM, 0)
     elif pow2:
         lg = int(math.log2(n))
         want = (STRATEGY_SIXSTEP, 1 << TUNED_SPLIT.get((lg, prec), lg // 2))

@@ -1586,6 +1586,20 @@ static int emit_axis_direct(Plan& p, int di, const AxisJob& j, std::string& algo
     if (is_pow2(j.n) && rows && j.n >= 16 && j.n * (prec ? 16 : 8) <= 512 &&
         !(p.desc.flags & AFFT_FLAG_MFMA))
         return emit_gen_single(p, di, j, algo);
+    // Long power-of-two columns, many side by side: 32 KiB of column and more
+    // leave the compile-time kernel fewer than 8 in a block, hence its two-pass
+    // form (emit_col_fourstep); the runtime-radix kernel holds 4 of 32 KiB in one
+    // pass.  Two passes -> one: complex128 2048 points, 256 columns 17.4 -> 11.4 us,
+    // 2048 51 -> 34, 4096 88 -> 64, 10000 258 -> 189; 4096 points, 1000 columns 51 -> 38;
+    // complex64 4096 points, 256 columns 17.6 -> 13.3, 4096 86 -> 77, 10000 269 -> 224.
+    // Not from 256 MiB on where the pitch is a multiple of 8 KiB: complex64 4096 x
+    // 8192 222 -> 280.
+    if (is_pow2(j.n) && j.in_cd == 1 && j.out_cd == 1 && j.in_nd >= j.count && j.out_nd >= j.count && j.count >= 128 &&
+        j.n * (prec ? 16 : 8) >= 32768 && gen_single_fits(prec, j.n, false) && !(p.desc.flags & AFFT_FLAG_MFMA)) {
+        const int64_t es = prec ? 16 : 8, pitch = std::max(j.in_nd, j.out_nd) * es;
+        if (xcd_order(j.in_nd * es, j.out_nd * es) || pitch * j.n < (int64_t(256) << 20))
+            return emit_gen_single(p, di, j, algo);
+    }
     if (is_pow2(j.n) && j.n <= max_single_pass(prec)) return emit_single(p, di, j, algo);
     if (is_pow2(j.n)) return emit_fourstep(p, di, j, algo);
     if (!smooth_schedule(j.n).empty()) {

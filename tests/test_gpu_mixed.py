@@ -216,3 +216,22 @@ def test_short_power_of_two_real_rows(ctx, n, batch, prec):
         p.inverse(y, X)
     assert rel_l2(X, O.rfft(x.astype(np.float64))) <= _tol(prec, n)
     assert rel_l2(y, O.irfft(X.astype(np.complex128), n)) <= _tol(prec, n)
+
+
+# long power-of-two columns: 128 side by side take one pass, fewer two
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("cols,pad", [(127, 0), (128, 0), (131, 0), (200, 5)])
+@pytest.mark.parametrize("n", [2048, 4096])
+def test_long_power_of_two_columns(ctx, n, cols, pad, prec, dt):
+    w = cols + pad
+    buf = synth.uniform_complex(n + cols, (n, w), dt)
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=cols, istride=w, idist=1, ostride=w, odist=1) as p:
+        if n * buf.itemsize >= 32768:
+            assert p.describe() == f"hip_mixed{n}c" if cols >= 128 else "colfourstep" in p.describe()
+        out = np.zeros_like(buf)
+        p.forward(out.ravel(), buf.ravel())
+        back = out.copy()
+        p.inverse(back.ravel(), back.ravel())   # in place
+    ref = O.fft_batch(np.ascontiguousarray(buf[:, :cols].T).astype(np.complex128)).T
+    assert rel_l2(out[:, :cols], ref) <= _tol(prec, n)
+    assert rel_l2(back[:, :cols], buf[:, :cols]) <= 2 * _tol(prec, n)
