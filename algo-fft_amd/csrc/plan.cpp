@@ -1318,17 +1318,27 @@ static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rade
 // 0.148; 1111 4096 0.164 -> 2268 0.150; 1313 4096 0.146 -> 2700 0.155; 2053 8192 0.354
 // -> 4200 0.191; 6001 16384 0.266 -> 12096 0.215.  2^23 complex128 points: 143 512 0.152
 // -> 288 0.114; 703 2048 0.135 -> 1440 0.124; 1529 4096 0.135 -> 3072 0.134; 2587 8192
-// 0.217 -> 5184 0.243.  Against the three-pass chain always, in up
+// 0.217 -> 5184 0.243.  It is also the quicker one through a few rows, up to so
+// many points of m: complex64 521, 2048 rows 13.3 against 15.2 us, 8192 44 against
+// 42; 2053, 256 rows 13.0 against 13.6, 512 24.6 against 16.1; complex128 521,
+// 1024 rows 14.6 against 17.2, 2048 26.4 against 23.2.  Against the three-pass chain always, in up
 // to four passes (complex64 8209 points 0.511 -> 0.239 ms, complex128 4099 0.530
 // -> 0.233), in more with rows enough: complex64 10007 on 20480 points in six
 // passes, 64 rows 0.041 -> 0.046, 256 0.068 -> 0.050.
 static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count, int64_t slices) {
     double factor = 1.0;
+    int64_t fewest = 0;
     if (m < 256) return 0;
     if (m <= max_single_pass(prec)) {
-        if (prec) factor = m <= 4096 ? 1.4 : 1.65;
-        else factor = m <= 1024 ? 1.45 : m <= 4096 ? 1.65 : 1.33;
+        if (prec) {
+            factor = m <= 1024 ? 1.4 : m <= 4096 ? 1.5 : 1.65;
+            if (m <= 4096) fewest = 1 << 23;
+        } else {
+            factor = m <= 1024 ? 1.45 : m <= 4096 ? 1.75 : 1.33;
+            fewest = m <= 4096 ? 1 << 24 : m <= 8192 ? 1 << 22 : 0;
+        }
     }
+    if (count * slices * m < fewest) return 0;
     int64_t best = 0;
     double least = 1e300;
     const int64_t top = std::min<int64_t>((int64_t)((double)m / factor), 163840 / (prec ? 16 : 8));
@@ -1356,14 +1366,20 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     // halves the points of the convolution: primes of 2^24 complex64 points, from
     // the padded form: 31 points 0.112 -> 0.106 ms, 257 0.215 -> 0.095, 1009 0.138
     // -> 0.091, 4051 0.24 -> 0.126, 8101 0.22 -> 0.144; 2^23 complex128: 61 0.115 -> 0.085,
-    // 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.
+    // 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.  A few rows are through the
+    // compile-time kernel sooner where m is 2048 or 4096 (complex64 1009: 64 rows
+    // 8.9 against 11.4 us, 1024 11.3 against 11.8, 2048 17.7 against 16.6; 2017: 512
+    // rows 11.5 against 14.5, 1024 18.2 against 17.6) or very short (17: 64
+    // rows 5.6 against 5.7).
     // Where the power of two is beyond LDS a row is one block's, the chain spreads
     // it over many: one launch from 64 rows on (complex128 4099 points, chain -> one
     // launch: 1 row 19.5 -> 25.7 us, 32 27.5 -> 26.3, 64 31.3 -> 26.7, 256 67 -> 33;
     // complex64 18433: 1 row 19.9 -> 41.5, 64 43.4 -> 42.8, 256 122 -> 52).
     if (!(p.desc.flags & AFFT_FLAG_REF_CHIRP) && (m <= max_single_pass(prec) || j.count * j.slices >= 64)) {
         MixShape ms;
-        if (p.desc.strategy != AFFT_STRATEGY_BLUESTEIN && n < 65536 && is_prime(n) && !smooth_schedule(n - 1).empty() &&
+        const int64_t fewest = m <= 128 ? 1 << 15 : m <= 1024 || m > 4096 ? 0 : 1 << 22;
+        if (p.desc.strategy != AFFT_STRATEGY_BLUESTEIN && j.count * j.slices * m >= fewest && n < 65536 &&
+            is_prime(n) && !smooth_schedule(n - 1).empty() &&
             mix_shape(n - 1, prec, MIX_ROWS, j.count, j.slices, ms, nullptr, 1))
             return emit_mix_blue(p, di, j, n - 1, true, algo);
         if (const int64_t sm = blue_smooth_length(n, m, prec, j.count, j.slices))

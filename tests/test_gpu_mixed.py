@@ -161,8 +161,9 @@ def test_short_power_of_two_rows(ctx, n, batch, prec, dt):
 def test_prime_rows(ctx, n, gap, prec, dt):
     if (n - 1) * (16 if prec else 8) > 163840:
         pytest.skip("longer rows take the three-pass chain")
-    # beyond a power of two in LDS the one-launch form starts at 64 rows
-    batch = 67 if n < 1000 or 2 * n - 1 > (8192 if prec else 16384) else 3
+    # enough rows for the one-launch form
+    m = 1 << (2 * n - 2).bit_length()
+    batch = (1 << 15) // m + 3 if m <= 128 else (1 << 22) // m + 3 if m <= 4096 else 67
     buf = synth.uniform_complex(n + gap, (batch, n + gap), dt)
     x = np.ascontiguousarray(buf[:, :n])
     ref = np.fft.fft(x.astype(np.complex128), axis=1)
@@ -191,7 +192,8 @@ def test_prime_rows(ctx, n, gap, prec, dt):
 @pytest.mark.parametrize("prec,dt", PRECS)
 @pytest.mark.parametrize("n", [22, 67, 69, 143, 341, 503, 703, 1111, 2053, 2587, 5117, 6002, 8209, 9797, 10201])
 def test_bluestein_rows_padded_to_smooth_lengths(ctx, n, prec, dt):
-    batch = 67 if n < 1000 or 2 * n - 1 > (8192 if prec else 16384) else 3
+    m = 1 << (2 * n - 2).bit_length()   # rows enough for the one-launch form
+    batch = (1 << 24) // m + 3 if m <= 4096 else 515
     x = synth.uniform_complex(n, (batch, n), dt)
     with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch) as p:
         got = np.empty_like(x)
