@@ -1728,8 +1728,10 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
     // compile-time kernel.  256 MiB of reals, compile-time -> runtime-radix
     // kernel, R2C / C2R: float32 32 points 0.196 / 0.179 -> 0.153 / 0.131 ms, 64 0.180 /
     // 0.148 -> 0.150 / 0.137; float64 32 0.175 / 0.212 -> 0.120 / 0.118.  128 points
-    // are mixed (R2C 0.140 -> 0.121, C2R 0.117 -> 0.133), 16 lose (0.158 -> 0.232).
-    const bool shortr = h == 16 || h == 32;
+    // are mixed (R2C 0.140 -> 0.121, C2R 0.117 -> 0.133), 16 lose (0.158 -> 0.232).  Under
+    // 1024 rows the compile-time kernel is quicker through (64 float32 points, 1 row
+    // 4.2 against 4.9 us).
+    const bool shortr = (h == 16 || h == 32) && rows * slices >= 1024;
     const KernelInfo* k = (h >= 2 && is_pow2(h) && !shortr) ? find_kernel(prec, (int)h, VAR_REAL, dir) : nullptr;
     if (k) {
         RArgs a{};

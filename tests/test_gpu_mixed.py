@@ -204,7 +204,8 @@ def test_bluestein_rows_padded_to_smooth_lengths(ctx, n, prec, dt):
     assert rel_l2(back, np.fft.ifft(got.astype(np.complex128), axis=1)) <= _tol(prec, n)
 
 
-# real rows of 32 and 64 points are this kernel's, their neighbours k_real's
+# real rows of 32 and 64 points are this kernel's from 1024 rows on, their
+# neighbours and fewer rows k_real's
 @pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
 @pytest.mark.parametrize("n", [16, 32, 64, 128])
 @pytest.mark.parametrize("batch", [1, 67, 4099])
