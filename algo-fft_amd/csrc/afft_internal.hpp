@@ -114,6 +114,7 @@ struct Plan {
     std::vector<Step> alias_steps[2];
     bool alias_same_ok[2] = {false, false};   // src == dst is safe without the copy
     size_t alias_bytes[2] = {0, 0};           // WORK2 bytes the copy needs
+    size_t alias_from[2] = {0, 0};            // steps[] from here on follow in alias_steps too
     std::vector<void*> owned;       // device tables
     size_t tmp_bytes[NTMP] = {0, 0, 0, 0};
     void* tmp[NTMP] = {nullptr, nullptr, nullptr, nullptr};

@@ -1793,8 +1793,32 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
             p.steps[di].push_back(s);
         }
         if (in_role == ROLE_SRC && out_role == ROLE_DST) {
+            // the same rows from a packed copy in WORK2, as large as the
+            // buffer of the two-launch form
+            const int64_t row = di ? h + 1 : h;
             p.alias_same_ok[di] = in_rd == out_rd && (slices == 1 || in_bd == out_bd);
-            p.alias_bytes[di] = (size_t)p.in_elems[di] * p.in_esize[di];
+            p.alias_bytes[di] = (size_t)(slices * rows * row * es);
+            std::vector<Step>& al = p.alias_steps[di];
+            const int64_t copies = rows == 1 ? 1 : slices;
+            for (int64_t y = 0; y < copies; ++y) {
+                Step cp = rows == 1 ? make_copy(prec, slices, row, in_bd, 1, row, 1, 1.0)
+                                    : make_copy(prec, rows, row, in_rd, 1, row, 1, 1.0);
+                cp.in_role = ROLE_SRC;
+                cp.in_off = y * in_bd * es;
+                cp.out_role = ROLE_WORK2;
+                cp.out_off = y * rows * row * es;
+                al.push_back(cp);
+            }
+            a.m.k.in_cd = row;
+            const size_t first = p.steps[di].size() - (size_t)slices;
+            for (int64_t y = 0; y < slices; ++y) {
+                Step s = p.steps[di][first + y];
+                std::memcpy(s.arg.data(), &a, sizeof(MixRealArgs));
+                s.in_role = ROLE_WORK2;
+                s.in_off = y * rows * row * es;
+                al.push_back(s);
+            }
+            p.alias_from[di] = p.steps[di].size();
         }
         if (!algo.empty()) algo += "+";
         algo += (di ? "c2r" : "r2c") + std::to_string(n);
@@ -2089,25 +2113,17 @@ int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
 // streaming loads alone lose.
 constexpr size_t kStreamOutBytes = size_t(128) << 20;
 
-static void build_alias_steps(Plan& p) {
-    const int prec = p.desc.precision;
-    for (int di = 0; di < 2; ++di) {
-        if (!p.alias_bytes[di]) continue;
-        Step c = make_copy(prec, 1, (int64_t)(p.alias_bytes[di] / (prec ? 16 : 8)), 0, 1, 0, 1, 1.0);
-        c.in_role = ROLE_SRC;
-        c.out_role = ROLE_WORK2;
-        p.alias_steps[di].push_back(c);
-        for (Step s : p.steps[di]) {
-            if (s.in_role == ROLE_SRC) s.in_role = ROLE_WORK2;
-            p.alias_steps[di].push_back(s);
-        }
-    }
+// The steps behind the fused real rows are the same for overlapping buffers.
+static void finish_alias_steps(Plan& p) {
+    for (int di = 0; di < 2; ++di)
+        if (!p.alias_steps[di].empty())
+            p.alias_steps[di].insert(p.alias_steps[di].end(), p.steps[di].begin() + p.alias_from[di], p.steps[di].end());
 }
 
 int build_plan(Plan& p) {
     int rc = build_plan_steps(p);
     if (rc) return rc;
-    build_alias_steps(p);
+    finish_alias_steps(p);
     for (int di = 0; di < 2; ++di) {
         const size_t ob = (size_t)p.out_elems[di] * p.out_esize[di];
         const size_t ib = (size_t)p.in_elems[di] * p.in_esize[di];

@@ -238,3 +238,30 @@ def test_long_power_of_two_columns(ctx, n, cols, pad, prec, dt):
     ref = O.fft_batch(np.ascontiguousarray(buf[:, :cols].T).astype(np.complex128)).T
     assert rel_l2(out[:, :cols], ref) <= _tol(prec, n)
     assert rel_l2(back[:, :cols], buf[:, :cols]) <= 2 * _tol(prec, n)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("direction", [A.FORWARD, A.INVERSE])
+def test_spread_real_rows_over_the_next_row(ctx, direction, noalloc):
+    """Rows far apart whose outputs lie over the next row's input: the copy
+    holds the rows alone, so it fits the static scratch although the rows'
+    extent (72 MB) does not."""
+    import ctypes
+    n, batch, pitch = 50, 300, 30000   # pitch in complex elements
+    h = n // 2
+    x = synth.uniform_real(n, (batch, n), np.float32)
+    X = np.fft.rfft(x.astype(np.float64), axis=1)
+    src = x.view(np.complex64) if direction == A.FORWARD else X.astype(np.complex64)
+    buf = torch.zeros((batch + 1, pitch), dtype=torch.complex64, device="cuda")
+    buf[:batch, :src.shape[1]] = torch.from_numpy(np.ascontiguousarray(src)).cuda()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    fn = A.lib().afft_plan_exec_device_noalloc if noalloc else A.lib().afft_plan_exec_device
+    with A.Plan.from_desc(ctx, (n,), kind=A.R2C, batch=batch, idist=2 * pitch, odist=pitch) as p:
+        A.check(fn(p.h, direction, ctypes.c_void_p(buf[1:].data_ptr()), ctypes.c_void_p(buf.data_ptr()),
+                   ctypes.c_void_p(s.cuda_stream)))
+        s.synchronize()
+    if direction == A.FORWARD:
+        assert rel_l2(buf[1:, :h + 1].cpu().numpy(), X) <= c64_tol(n)
+    else:
+        assert rel_l2(np.ascontiguousarray(buf[1:, :h].cpu().numpy()).view(np.float32), x) <= 2 * c64_tol(n)
