@@ -108,9 +108,10 @@ struct Plan {
     int out_esize[2] = {0, 0};
     std::vector<Step> steps[2];     // [0] forward, [1] inverse
     // Steps of a direction whose first launch may not write over its input
-    // while other blocks still read it (fused real rows, whose two sides have
-    // different row lengths): the input is copied to WORK2 first.  Used when
-    // the caller's src and dst overlap (alias_steps_for); empty otherwise.
+    // while other blocks still read it: fused real rows, whose two sides have
+    // different row lengths, and single launches where other lengths go
+    // through scratch.  The input is copied to WORK2 first.  Used when the
+    // caller's src and dst overlap (steps_for); empty otherwise.
     std::vector<Step> alias_steps[2];
     bool alias_same_ok[2] = {false, false};   // src == dst is safe without the copy
     size_t alias_bytes[2] = {0, 0};           // WORK2 bytes the copy needs
@@ -157,7 +158,7 @@ MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw);
 struct BlueTables {
     const void* chirp = nullptr;                 // n entries, forward sign
     const void* filt[2] = {nullptr, nullptr};    // [fwd, inv], m entries, 1/m folded in
-    const void* post[2] = {nullptr, nullptr};    // [fwd, inv]: chirp, conj(chirp)*inv_scale
+    const void* post[2] = {nullptr, nullptr};    // [fwd, inv]: chirp, conj(chirp)*inv_scale (none at inv_scale 0)
     const void* perm = nullptr;                  // Rader: g^q mod n, uint16
 };
 // tr_m1 > 0 stores the filter spectra row-major as [k1][k2], k = k1 + tr_m1*k2

@@ -15,6 +15,7 @@
 
 #include <cmath>
 #include <complex>
+#include <memory>
 
 #include "afft_internal.hpp"
 #include "kblue.hpp"
@@ -1128,12 +1129,12 @@ static bool is_prime(int64_t n) {
 int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt, int64_t tr_m1) {
     const bool refchirp = p.desc.flags & AFFT_FLAG_REF_CHIRP;
     int rc;
-    auto up = [&](const std::vector<double>& v, const void** dev) -> int {
+    auto up = [&](const double* v, int64_t len, const void** dev) -> int {
         if (p.desc.precision == 0) {
-            std::vector<float> f(v.begin(), v.end());
+            std::vector<float> f(v, v + len);
             return upload_table(p, f.data(), f.size() * 4, dev);
         }
-        return upload_table(p, v.data(), v.size() * 8, dev);
+        return upload_table(p, v, (size_t)len * 8, dev);
     };
     // chirp and filter spectra are shared by the plan's two directions
     const auto key = std::make_tuple(n, m, tr_m1);
@@ -1192,13 +1193,13 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
         } else if ((rc = device_fft_c128(p, spec, m))) {
             return rc;
         }
-        std::vector<double> filt[2];
+        std::unique_ptr<double[]> filt[2];   // not cleared: every entry is written once
         // natural order, or row-major [k1][k2] of k = k1 + tr_m1 * k2
         const int64_t m2 = tr_m1 > 0 ? m / tr_m1 : 0;
         const double dm = (double)m, inv_m = 1.0 / dm;
         const bool exact = is_pow2(m);   // then x * inv_m == x / m, and far cheaper
         auto div = [&](double x) { return exact ? x * inv_m : x / dm; };
-        for (int d = 0; d < 2; ++d) filt[d].resize(2 * m);
+        for (int d = 0; d < 2; ++d) filt[d].reset(new double[2 * m]);
         // filt[0][at] = spec[k] / m, filt[1][at] = conj(spec[-k mod m]) / m,
         // through a buffer where the order changes (runs of 32 points read,
         // of 256 points written)
@@ -1234,9 +1235,9 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
         } else {
             for (int64_t k = 0; k < m; ++k) put(&spec[2 * k], &spec[k ? 2 * (m - k) : 0], k);
         }
-        if (tr_m1 != BLUE_RADER && (rc = up(bc.ch, &bc.chirp))) return rc;
+        if (tr_m1 != BLUE_RADER && (rc = up(bc.ch.data(), 2 * n, &bc.chirp))) return rc;
         for (int d = 0; d < 2; ++d)
-            if ((rc = up(filt[d], &bc.filt[d]))) return rc;
+            if ((rc = up(filt[d].get(), 2 * m, &bc.filt[d]))) return rc;
         it = p.blue_cache.emplace(key, std::move(bc)).first;
     }
     const std::vector<double>& ch = it->second.ch;
@@ -1248,14 +1249,16 @@ int blue_tables(Plan& p, int64_t n, int64_t m, double inv_scale, BlueTables& bt,
     // post-multiply tables: the chirp itself (forward), conj(chirp) times the
     // inverse scale (inverse)
     bt.post[0] = bt.chirp;
+    if (inv_scale == 0.0) return AFFT_OK;
     std::vector<double> post(2 * n);
     for (int64_t k = 0; k < n; ++k) {
         post[2 * k] = ch[2 * k] * inv_scale;
         post[2 * k + 1] = -ch[2 * k + 1] * inv_scale;
     }
-    return up(post, &bt.post[1]);
+    return up(post.data(), 2 * n, &bt.post[1]);
 }
 
+static void alias_through_copy(Plan& p, int di, const AxisJob& j);
 const void* mix_blue_kernel_c64();
 const void* mix_blue_kernel_c128();
 const void* mix_rader_kernel_c64();
@@ -1269,7 +1272,7 @@ static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rade
     BlueTables bt;
     MixBlueArgs a{};
     MixShape ms;
-    int rc = blue_tables(p, j.n, m, 1.0, bt, rader ? BLUE_RADER : 0);
+    int rc = blue_tables(p, j.n, m, 0.0, bt, rader ? BLUE_RADER : 0);
     if (rc || (rc = mix_args(p, m, MIX_ROWS, j.count, j.slices, a.m, ms, rader ? 1 : 0))) return rc;
     const void* fn = rader ? (prec ? mix_rader_kernel_c128() : mix_rader_kernel_c64())
                            : (prec ? mix_blue_kernel_c128() : mix_blue_kernel_c64());
@@ -1301,6 +1304,7 @@ static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rade
         s.name = name;
         p.steps[di].push_back(s);
     }
+    if (next_pow2(2 * j.n - 1) > max_single_pass(prec)) alias_through_copy(p, di, j);
     if (!algo.empty()) algo += "+";
     algo += name + (rader ? "" : "m" + std::to_string(m));
     return AFFT_OK;
@@ -1387,7 +1391,7 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     }
     if (m <= max_single_pass(prec)) {
         BlueTables bt;
-        int rc = blue_tables(p, n, m, 1.0, bt);
+        int rc = blue_tables(p, n, m, 0.0, bt);
         if (rc) return rc;
         const KernelInfo* k = find_kernel(prec, (int)m, VAR_BLUE, dir);
         if (!k) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "no Bluestein kernel for M=" + std::to_string(m));
@@ -1445,7 +1449,7 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     if (!ka || !kr || !kc) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "missing Bluestein chain kernel");
     BlueTables bt;
     // the inverse scale rides on the post-multiply table
-    int rc = blue_tables(p, n, m, di ? j.scale : 1.0, bt, m1);
+    int rc = blue_tables(p, n, m, di ? j.scale : 0.0, bt, m1);
     if (rc) return rc;
     // chunks of transforms whose M-point intermediate stays in the last-level
     // cache between the three passes
@@ -1522,6 +1526,32 @@ static Step make_copy(int prec, int64_t lines, int64_t len, int64_t icd, int64_t
 }
 
 static int emit_axis_direct(Plan& p, int di, const AxisJob& j, std::string& algo);
+
+// The last step is one launch from the caller's input to its output where
+// other lengths take several through scratch.  Where src and dst overlap and
+// are not the same rows, it reads a packed copy instead (alias_steps): blocks
+// would overwrite what others have yet to read.
+static void alias_through_copy(Plan& p, int di, const AxisJob& j) {
+    if (p.desc.rank != 1 || j.slices != 1 || j.in_role != ROLE_SRC || j.out_role != ROLE_DST) return;
+    const bool rows = j.in_nd == 1;
+    Step c = make_copy(p.desc.precision, j.count, j.n, j.in_cd, j.in_nd, rows ? j.n : 1, rows ? 1 : j.count, 1.0);
+    c.in_role = ROLE_SRC;
+    c.in_off = j.in_off;
+    c.out_role = ROLE_WORK2;
+    Step s = p.steps[di].back();
+    KArgs k;   // first in every argument block of k_mix's kernels
+    std::memcpy(&k, s.arg.data(), sizeof(k));
+    k.in_cd = rows ? j.n : 1;
+    k.in_nd = rows ? 1 : j.count;
+    std::memcpy(s.arg.data(), &k, sizeof(k));
+    s.in_role = ROLE_WORK2;
+    s.in_off = 0;
+    p.alias_steps[di] = {c, s};
+    p.alias_from[di] = p.steps[di].size();
+    p.alias_same_ok[di] = j.in_cd == j.out_cd && j.in_nd == j.out_nd;
+    p.alias_bytes[di] = (size_t)(j.count * j.n) * (p.desc.precision ? 16 : 8);
+}
+static_assert(offsetof(MixArgs, k) == 0 && offsetof(MixBlueArgs, m) == 0, "KArgs first");
 
 // Paths that need unit-stride rows get strided lines through a gather into
 // TMP1, the row transform in place there, and a scatter back.
@@ -1613,8 +1643,11 @@ static int emit_axis_direct(Plan& p, int di, const AxisJob& j, std::string& algo
     if (is_pow2(j.n) && j.in_cd == 1 && j.out_cd == 1 && j.in_nd >= j.count && j.out_nd >= j.count && j.count >= 128 &&
         j.n * (prec ? 16 : 8) >= 32768 && gen_single_fits(prec, j.n, false) && !(p.desc.flags & AFFT_FLAG_MFMA)) {
         const int64_t es = prec ? 16 : 8, pitch = std::max(j.in_nd, j.out_nd) * es;
-        if (xcd_order(j.in_nd * es, j.out_nd * es) || pitch * j.n < (int64_t(256) << 20))
-            return emit_gen_single(p, di, j, algo);
+        if (xcd_order(j.in_nd * es, j.out_nd * es) || pitch * j.n < (int64_t(256) << 20)) {
+            const int rc = emit_gen_single(p, di, j, algo);
+            if (rc == AFFT_OK) alias_through_copy(p, di, j);
+            return rc;
+        }
     }
     if (is_pow2(j.n) && j.n <= max_single_pass(prec)) return emit_single(p, di, j, algo);
     if (is_pow2(j.n)) return emit_fourstep(p, di, j, algo);

@@ -343,7 +343,7 @@ static int ragged_build(afft_ragged_s& r) {
                 BlueTables bt;
                 r.tables.desc.precision = r.prec;
                 r.tables.desc.flags = r.flags;
-                if ((rc = blue_tables(r.tables, n, m, 1.0, bt, key.second))) return rc;
+                if ((rc = blue_tables(r.tables, n, m, 0.0, bt, key.second))) return rc;
                 it = bcache.emplace(key, bt).first;
             }
             j.chirp = it->second.chirp;

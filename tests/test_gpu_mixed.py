@@ -265,3 +265,44 @@ def test_spread_real_rows_over_the_next_row(ctx, direction, noalloc):
         assert rel_l2(buf[1:, :h + 1].cpu().numpy(), X) <= c64_tol(n)
     else:
         assert rel_l2(np.ascontiguousarray(buf[1:, :h].cpu().numpy()).view(np.float32), x) <= 2 * c64_tol(n)
+
+
+# single launches where other lengths go through scratch: dst over src with
+# other distances between the rows or columns
+@pytest.mark.parametrize("prec,dt", PRECS)
+@pytest.mark.parametrize("kind", ["rows", "columns"])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_other_distances_over_the_input(ctx, kind, noalloc, prec, dt):
+    import ctypes
+    if kind == "rows":   # Rader's form, its power of two beyond LDS
+        n, batch = (12289 if prec == A.COMPLEX64 else 4201), 70
+        lay = dict(idist=n, odist=n + 5)
+    else:
+        n, batch = (4096 if prec == A.COMPLEX64 else 2048), 130
+        lay = dict(istride=batch, idist=1, ostride=batch + 5, odist=1)
+    x = synth.uniform_complex(n, (batch, n), dt)
+    ref = np.fft.fft(x.astype(np.complex128), axis=1)
+    buf = torch.zeros(batch * n + 5 * max(n, batch), dtype=torch.from_numpy(x[:1]).dtype, device="cuda")
+    buf[:batch * n] = torch.from_numpy(np.ascontiguousarray(x if kind == "rows" else x.T).ravel()).cuda()
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    fn = A.lib().afft_plan_exec_device_noalloc if noalloc else A.lib().afft_plan_exec_device
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch, **lay) as p:
+        assert p.describe() in (f"hip_rader{n}", f"hip_mixed{n}c")
+        for i in range(2):
+            A.check(fn(p.h, A.FORWARD if i == 0 else A.INVERSE, ctypes.c_void_p(buf.data_ptr()),
+                       ctypes.c_void_p(buf.data_ptr()), ctypes.c_void_p(s.cuda_stream)))
+            s.synchronize()
+            if i == 0:
+                y = buf.cpu().numpy()
+                got = (y[:batch * (n + 5)].reshape(batch, n + 5)[:, :n] if kind == "rows"
+                       else y[:n * (batch + 5)].reshape(n, batch + 5)[:, :batch].T)
+                assert rel_l2(got, ref) <= _tol(prec, n)
+                # the inverse reads the plan's input layout
+                z = np.ascontiguousarray(got if kind == "rows" else got.T)
+                buf[:batch * n] = torch.from_numpy(z.ravel()).cuda()
+                torch.cuda.synchronize()
+    y = buf.cpu().numpy()
+    got = (y[:batch * (n + 5)].reshape(batch, n + 5)[:, :n] if kind == "rows"
+           else y[:n * (batch + 5)].reshape(n, batch + 5)[:, :batch].T)
+    assert rel_l2(got, x) <= 2 * _tol(prec, n)
