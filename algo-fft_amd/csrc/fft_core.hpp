@@ -66,7 +66,8 @@ struct LdsCol {
     __device__ __forceinline__ int operator()(int n) const { return n * TPB + c; }
 };
 
-template <typename T, class S, int E, int DIR, int p, bool HOIST, class TW, class L>
+// XCHG false: the exchange through LDS is the caller's (core_planar).
+template <typename T, class S, int E, int DIR, int p, bool HOIST, bool XCHG = true, class TW, class L>
 __device__ __forceinline__ void core_pass(cx<T> (&v)[E], cx<T>* lds, int t, TW tw, const L& li) {
     constexpr int N = S::N;
     constexpr int TT = N / E;
@@ -99,7 +100,7 @@ __device__ __forceinline__ void core_pass(cx<T> (&v)[E], cx<T>* lds, int t, TW t
         }
     };
     if constexpr (NS > 1 && HOIST) load_tw();
-    if constexpr (p > 0) {
+    if constexpr (p > 0 && XCHG) {
         __syncthreads();
 #pragma unroll
         for (int b = 0; b < B; ++b)
@@ -134,7 +135,7 @@ __device__ __forceinline__ void core_pass(cx<T> (&v)[E], cx<T>* lds, int t, TW t
     }
 #pragma unroll
     for (int b = 0; b < B; ++b) dft<R, DIR, B>(v + b);
-    if constexpr (p < S::P - 1) {
+    if constexpr (p < S::P - 1 && XCHG) {
         if constexpr (p > 0) __syncthreads();
 #pragma unroll
         for (int b = 0; b < B; ++b) {
@@ -176,6 +177,48 @@ __device__ __forceinline__ void core_turn(cx<T> (&v)[E], cx<T>* lds, int t, TW t
     static_assert(S::P > 1, "one pass exchanges nothing");
     core_head<T, S, E, DIR>(v, lds, t, tw, li, std::make_integer_sequence<int, S::P - 1>{});
     core_pass<T, S, E, DIR, S::P - 1, false>(v, lds, tl, tw, ll);
+}
+
+// The exchange between passes p and p + 1 through half the LDS: the real parts
+// of all points, then the imaginary parts in the same place.
+template <typename T, class S, int E, int p, class L>
+__device__ __forceinline__ void planar_exchange(cx<T> (&v)[E], T* lds, int t, const L& li) {
+    constexpr int TT = S::N / E, R = S::rad[p], NS = S::ns(p), B = E / R, R2 = S::rad[p + 1], B2 = E / R2;
+    auto put = [&](auto part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int j = t + TT * b;
+            const int base = (j / NS) * NS * R + (j % NS);
+#pragma unroll
+            for (int r = 0; r < R; ++r) lds[li(base + r * NS)] = part(v[b + r * B]);
+        }
+    };
+    auto get = [&](auto part) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < B2; ++b)
+#pragma unroll
+            for (int r = 0; r < R2; ++r) part(v[b + r * B2]) = lds[li(t + TT * b + r * (S::N / R2))];
+    };
+    auto re = [](cx<T>& z) -> T& { return z.x; };
+    auto im = [](cx<T>& z) -> T& { return z.y; };
+    if constexpr (p > 0) __syncthreads();
+    put(re);
+    __syncthreads();
+    get(re);
+    __syncthreads();
+    put(im);
+    __syncthreads();
+    get(im);
+}
+
+// core with planar exchanges: half the LDS for twice the barriers.
+template <typename T, class S, int E, int DIR, int p, class TW, class L>
+__device__ __forceinline__ void core_planar(cx<T> (&v)[E], T* lds, int t, TW tw, const L& li) {
+    core_pass<T, S, E, DIR, p, false, false>(v, (cx<T>*)nullptr, t, tw, li);
+    if constexpr (p < S::P - 1) {
+        planar_exchange<T, S, E, p>(v, lds, t, li);
+        core_planar<T, S, E, DIR, p + 1>(v, lds, t, tw, li);
+    }
 }
 
 }  // namespace afft

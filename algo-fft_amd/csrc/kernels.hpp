@@ -68,6 +68,20 @@ struct KCfg {
     static constexpr int LDS_ELEMS = S::P > 1 || VAR == VAR_4B
                                          ? (ROWL ? TPB * LdsRow<N, PADSH>::SLAB : TPB * N)
                                          : 1;
+    // Whether k_fft has a second form of this kernel with planar exchanges
+    // (planar_exchange): 64 KiB of LDS a block instead of 128, so that one block
+    // loads and stores while the other computes.
+    // Taken from two blocks a CU on (make_step).  complex128 rows of 8192
+    // points, 4096 rows 0.228 -> 0.188 ms, 512 33.7 -> 28.4 us; columns of 1024
+    // complex64 points, 64 x 1024 x 1000 0.457 -> 0.431 ms, 16 real images of 1024 x
+    // 1024 63 -> 60 us; of 512 complex128, 16 x 512 x 500 52 -> 48 us, 1,000,003 points x
+    // 8 0.383 -> 0.365 ms (line-aligned pitches come out even).
+    // Other kernels of that size lose by the barriers: complex64 rows of 16384
+    // 0.238 -> 0.272, transposing rows (2^20 complex64 0.448 -> 0.479), four-step
+    // columns (2^18 complex128 0.208 -> 0.215, 2^22 complex64 0.566 -> 0.602), columns of
+    // 512 (0.566 -> 0.570) and 2048 complex64 (0.433 -> 0.441).
+    static constexpr bool PLANAR = sizeof(T) == 4 ? VAR == VAR_COL && N == 1024
+                                                  : (VAR == VAR_ROW && N == 8192) || (VAR == VAR_COL && N == 512);
 };
 
 // Forward-sign W_L^m from the two-level table; callers conjugate for DIR=+1.
@@ -92,12 +106,13 @@ __device__ __forceinline__ void xcd_block(unsigned* bx, unsigned* by) {
     *bx = nl - *by * gridDim.x;
 }
 
-template <typename T, class S, int E, int TPB, int VAR, int DIR>
+template <typename T, class S, int E, int TPB, int VAR, int DIR, bool PLANAR = false>
 __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArgs a) {
     using C = KCfg<T, S, E, TPB, VAR>;
     constexpr int N = S::N;
     constexpr int TT = C::TT;
-    __shared__ cx<T> lds[C::LDS_ELEMS];
+    using Slot = std::conditional_t<PLANAR, T, cx<T>>;
+    __shared__ Slot lds[C::LDS_ELEMS];
     const int tid = threadIdx.x;
     int c, t;
     if constexpr (C::ROWL) { c = tid / TT; t = tid % TT; }
@@ -141,7 +156,11 @@ __global__ void __launch_bounds__((KCfg<T, S, E, TPB, VAR>::THREADS)) k_fft(KArg
 
     // VAR_4B stores with lanes along c: transform c2, thread t2 of it
     const int c2 = tid % TPB, t2 = tid / TPB;
-    if constexpr (VAR == VAR_4B && S::P > 1) {
+    if constexpr (PLANAR && C::ROWL) {
+        core_planar<T, S, E, DIR, 0>(v, lds, t, tw, LdsRow<N, C::PADSH>(c));
+    } else if constexpr (PLANAR) {
+        core_planar<T, S, E, DIR, 0>(v, lds, t, tw, LdsCol<TPB>(c));
+    } else if constexpr (VAR == VAR_4B && S::P > 1) {
         // The last pass already runs with lanes along c: without a trip
         // through LDS of its own for the store, 512 MiB of complex64 2^20
         // 0.464 -> 0.448 ms, 65536 0.362 -> 0.358, 2^22 0.583 -> 0.566,
@@ -496,6 +515,7 @@ enum { KIND_FFT = 0, KIND_BLUE = 1, KIND_REAL = 2 };
 
 struct KernelInfo {
     const void* fn;
+    const void* planar;   // k_fft with planar exchanges, or null
     int kind;       // KIND_FFT (k_fft) or KIND_BLUE (k_blue)
     int prec;       // 0 = complex64, 1 = complex128
     int n;
@@ -527,6 +547,7 @@ struct Registrar {
             k.kind = KIND_REAL;
         } else {
             k.fn = (const void*)&k_fft<T, S, E, TPB, VAR, DIR>;
+            if constexpr (C::PLANAR) k.planar = (const void*)&k_fft<T, S, E, TPB, VAR, DIR, true>;
             k.kind = KIND_FFT;
         }
         k.prec = sizeof(T) == 4 ? 0 : 1;

@@ -306,3 +306,31 @@ def test_other_distances_over_the_input(ctx, kind, noalloc, prec, dt):
     got = (y[:batch * (n + 5)].reshape(batch, n + 5)[:, :n] if kind == "rows"
            else y[:n * (batch + 5)].reshape(n, batch + 5)[:, :batch].T)
     assert rel_l2(got, x) <= 2 * _tol(prec, n)
+
+
+# k_fft's planar exchanges (two blocks a CU and more) against numpy, the last
+# block partial
+@pytest.mark.parametrize("kind,n,prec", [("rows", 8192, A.COMPLEX128), ("columns", 1024, A.COMPLEX64),
+                                         ("columns", 512, A.COMPLEX128)])
+@pytest.mark.parametrize("direction", [A.FORWARD, A.INVERSE])
+def test_planar_exchange(ctx, kind, n, prec, direction):
+    dt = torch.complex64 if prec == A.COMPLEX64 else torch.complex128
+    batch = 515 if kind == "rows" else 512 * 16 + 5   # 16 columns a block
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn((batch, n) if kind == "rows" else (n, batch), generator=g, device="cuda", dtype=dt)
+    y = torch.empty_like(x)
+    lay = {} if kind == "rows" else dict(istride=batch, idist=1, ostride=batch, odist=1)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with A.Plan.from_desc(ctx, (n,), precision=prec, batch=batch, **lay) as p:
+        assert p.describe() == f"hip_lds{n}" + kind[0]
+        p.exec_device(direction, y.data_ptr(), x.data_ptr(), s.cuda_stream)
+        s.synchronize()
+    fft = np.fft.fft if direction == A.FORWARD else np.fft.ifft
+    ref = fft(x.cpu().numpy().astype(np.complex128), axis=1 if kind == "rows" else 0)
+    got = y.cpu().numpy()
+    assert rel_l2(got, ref) <= _tol(prec, n)
+    if kind == "rows":
+        assert rel_l2(got[-1], ref[-1]) <= _tol(prec, n)
+    else:
+        assert rel_l2(got[:, -5:], ref[:, -5:]) <= _tol(prec, n)
