@@ -97,6 +97,8 @@ struct BlueCache {
     const void* perm = nullptr;
 };
 
+struct MixCache;   // plan.cpp
+
 struct Plan {
     Context* ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -116,6 +118,7 @@ struct Plan {
     bool alias_same_ok[2] = {false, false};   // src == dst is safe without the copy
     size_t alias_bytes[2] = {0, 0};           // WORK2 bytes the copy needs
     size_t alias_from[2] = {0, 0};            // steps[] from here on follow in alias_steps too
+    std::shared_ptr<MixCache> mix_cache;   // launch shapes and tables already made
     std::vector<void*> owned;       // device tables
     size_t tmp_bytes[NTMP] = {0, 0, 0, 0};
     void* tmp[NTMP] = {nullptr, nullptr, nullptr, nullptr};
