@@ -1503,7 +1503,7 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
     if ((rc = schedule_twiddles(p, kc, &C.tw))) return rc;
     C.count = m2;
     C.in_cd = C.out_cd = 1; C.in_nd = C.out_nd = m2; C.in_bd = m; C.out_bd = j.out_cd;
-    C.scale = 1.0;
+    C.scale = di ? 1.0 : j.scale;   // normalised and unitary forward plans
     C.xcd = A.xcd;
     C.fuse = FUSE_CROP_OUT;
     C.fvec = bt.post[di];
