@@ -113,14 +113,15 @@ struct Plan {
     // while other blocks still read it: fused real rows, whose two sides have
     // different row lengths, and single launches where other lengths go
     // through scratch.  The input is copied to WORK2 first.  Used when the
-    // caller's src and dst overlap (steps_for); empty otherwise.
+    // caller's src and dst overlap (launches_for); empty otherwise.
     std::vector<Step> alias_steps[2];
     bool alias_same_ok[2] = {false, false};   // src == dst is safe without the copy
     size_t alias_bytes[2] = {0, 0};           // WORK2 bytes the copy needs
     size_t alias_from[2] = {0, 0};            // steps[] from here on follow in alias_steps too
+    bool alias_reserved = false;              // reserve_alias has run
     std::shared_ptr<MixCache> mix_cache;   // launch shapes and tables already made
     std::vector<void*> owned;       // device tables
-    size_t tmp_bytes[NTMP] = {0, 0, 0, 0};
+    size_t tmp_bytes[NTMP] = {0, 0, 0, 0};   // what steps[] use; fixed once the plan is built
     void* tmp[NTMP] = {nullptr, nullptr, nullptr, nullptr};
     void* stage_in = nullptr;
     void* stage_out = nullptr;
@@ -191,9 +192,19 @@ bool parse_strategy(const std::string& algo, Candidate* c);
 // Predicted log-runtimes of candidates (GPU inference); 0 on success.
 int mlp_predict_host(Mlp* m, const float* x, int64_t n, float* y);
 int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s);
-// Steps to run for these buffers: the direction's own, or its aliasing ones
-// where src and dst overlap (the plan's WORK2 size is raised to what they need).
-std::vector<Step>& steps_for(Plan& p, int di, const void* dst, const void* src);
+// The launches of direction di for these buffers, the direction's own or its
+// aliasing ones where src and dst overlap, and the workspace that they use.
+struct Launches {
+    std::vector<Step>& steps;
+    size_t bytes[NTMP];
+};
+Launches launches_for(Plan& p, int di, const void* dst, const void* src);
+// Bytes of workspace buffer t as it is allocated: what either kind of launches uses.
+size_t buffer_bytes(const Plan& p, int t);
+// The first execution of a plan with aliasing launches outside stream capture
+// allocates their buffer too, so that a later call over its input may be
+// captured (rows with a copy beyond kRowAliasReserve excepted).
+int reserve_alias(Plan& p, hipStream_t s);
 // Enqueues steps with explicit workspace buffers; allocates nothing and
 // records no event.
 int launch_steps(std::vector<Step>& steps, void* dst, const void* src, void* const* tmp, hipStream_t s);

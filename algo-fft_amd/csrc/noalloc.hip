@@ -33,11 +33,11 @@ std::mutex g_mu;
 void* g_ptr[kMaxDevices] = {};
 
 // Byte offset of each scratch role inside the array, 256-byte aligned.
-size_t carve(const Plan& p, size_t off[NTMP]) {
+size_t carve(const size_t bytes[NTMP], size_t off[NTMP]) {
     size_t total = 0;
     for (int t = 0; t < NTMP; ++t) {
         off[t] = total;
-        total += (p.tmp_bytes[t] + 255) & ~size_t(255);
+        total += (bytes[t] + 255) & ~size_t(255);
     }
     return total;
 }
@@ -81,9 +81,9 @@ int afft_plan_exec_device_noalloc(afft_plan p, int direction, void* dst, const v
     const int di = direction == AFFT_INVERSE ? 1 : 0;
     if (p->steps[di].empty()) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "direction not available for this plan kind");
     std::lock_guard<std::mutex> lock(p->mu);
-    std::vector<Step>& steps = steps_for(*p, di, dst, src);
+    const Launches l = launches_for(*p, di, dst, src);
     size_t off[NTMP];
-    const size_t need = carve(*p, off);
+    const size_t need = carve(l.bytes, off);
     if (need > kNoAllocScratchBytes)
         return set_error(AFFT_ERR_INVALID_LENGTH, "plan needs " + std::to_string(need) +
                                                       " bytes of scratch; the static scratch holds " +
@@ -93,8 +93,8 @@ int afft_plan_exec_device_noalloc(afft_plan p, int direction, void* dst, const v
     if (rc) return rc;
     AFFT_HIP(hipSetDevice(p->ctx->device));
     void* tmp[NTMP];
-    for (int t = 0; t < NTMP; ++t) tmp[t] = p->tmp_bytes[t] ? (char*)base + off[t] : nullptr;
-    rc = launch_steps(steps, dst, src, tmp, stream ? (hipStream_t)stream : p->stream);
+    for (int t = 0; t < NTMP; ++t) tmp[t] = l.bytes[t] ? (char*)base + off[t] : nullptr;
+    rc = launch_steps(l.steps, dst, src, tmp, stream ? (hipStream_t)stream : p->stream);
     if (rc == AFFT_OK) clear_error();
     return rc;
 }

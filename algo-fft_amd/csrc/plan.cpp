@@ -2100,16 +2100,41 @@ static int build_plan_steps(Plan& p) {
     return AFFT_OK;
 }
 
-std::vector<Step>& steps_for(Plan& p, int di, const void* dst, const void* src) {
-    if (p.alias_steps[di].empty() || (src == dst && p.alias_same_ok[di])) return p.steps[di];
+Launches launches_for(Plan& p, int di, const void* dst, const void* src) {
     const char* s0 = (const char*)src;
     const char* d0 = (const char*)dst;
     const bool apart = s0 + (size_t)p.in_elems[di] * p.in_esize[di] <= d0 ||
                        d0 + (size_t)p.out_elems[di] * p.out_esize[di] <= s0;
-    if (apart) return p.steps[di];
-    size_t& w = p.tmp_bytes[ROLE_WORK2 - 2];
-    w = std::max({w, p.alias_bytes[0], p.alias_bytes[1]});
-    return p.alias_steps[di];
+    const bool own = p.alias_steps[di].empty() || apart || (src == dst && p.alias_same_ok[di]);
+    Launches l{own ? p.steps[di] : p.alias_steps[di], {}};
+    std::copy(p.tmp_bytes, p.tmp_bytes + NTMP, l.bytes);
+    if (!own) l.bytes[ROLE_WORK2 - 2] = std::max(l.bytes[ROLE_WORK2 - 2], p.alias_bytes[di]);
+    return l;
+}
+
+size_t buffer_bytes(const Plan& p, int t) {
+    return t == ROLE_WORK2 - 2 ? std::max({p.tmp_bytes[t], p.alias_bytes[0], p.alias_bytes[1]}) : p.tmp_bytes[t];
+}
+
+// Rows whose other route takes its scratch in chunks (fourstep_chunk_bytes):
+// a longer copy is allocated by the first call that needs it.  The other
+// routes of real rows and of columns hold the whole batch.
+constexpr size_t kRowAliasReserve = size_t(128) << 20;
+
+int reserve_alias(Plan& p, hipStream_t s) {
+    constexpr int t = ROLE_WORK2 - 2;
+    if (p.alias_reserved || p.tmp[t] || buffer_bytes(p, t) == p.tmp_bytes[t]) return AFFT_OK;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    AFFT_HIP(hipStreamIsCapturing(s, &cs));
+    if (cs != hipStreamCaptureStatusNone) return AFFT_OK;
+    p.alias_reserved = true;
+    if (p.desc.kind == AFFT_C2C && p.desc.istride <= 1 && buffer_bytes(p, t) > kRowAliasReserve) return AFFT_OK;
+    // without the memory only calls over their input fail, when they ask for it
+    if (hipMalloc(&p.tmp[t], buffer_bytes(p, t)) != hipSuccess) {
+        (void)hipGetLastError();
+        p.tmp[t] = nullptr;
+    }
+    return AFFT_OK;
 }
 
 // Enqueues steps on s, with the roles resolved to src, dst and the workspace
@@ -2135,12 +2160,12 @@ int launch_steps(std::vector<Step>& steps, void* dst, const void* src, void* con
 // touched.
 int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
     const int di = dir == AFFT_INVERSE ? 1 : 0;
-    std::vector<Step>& steps = steps_for(p, di, dst, src);
+    const Launches l = launches_for(p, di, dst, src);
     bool ws = false;
     for (int t = 0; t < NTMP; ++t) {
-        if (!p.tmp_bytes[t]) continue;
+        if (!l.bytes[t]) continue;
         ws = true;
-        if (!p.tmp[t]) AFFT_HIP(hipMalloc(&p.tmp[t], p.tmp_bytes[t]));
+        if (!p.tmp[t]) AFFT_HIP(hipMalloc(&p.tmp[t], buffer_bytes(p, t)));
     }
     if (ws) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2152,7 +2177,7 @@ int exec_plan(Plan& p, int dir, void* dst, const void* src, hipStream_t s) {
             if (p.ws_used && p.ws_stream != s) AFFT_HIP(hipStreamWaitEvent(s, p.ws_done, 0));
         }
     }
-    int rc = launch_steps(steps, dst, src, p.tmp, s);
+    int rc = launch_steps(l.steps, dst, src, p.tmp, s);
     if (rc) return rc;
     if (ws) {
         AFFT_HIP(hipEventRecord(p.ws_done, s));

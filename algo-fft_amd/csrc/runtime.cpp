@@ -694,7 +694,9 @@ int afft_plan_exec_device(afft_plan p, int direction, void* dst, const void* src
         return set_error(AFFT_ERR_NOT_IMPLEMENTED, "direction not available for this plan kind");
     std::lock_guard<std::mutex> lock(p->mu);
     AFFT_HIP(hipSetDevice(p->ctx->device));
-    int rc = exec_plan(*p, direction, dst, src, stream ? (hipStream_t)stream : p->stream);
+    const hipStream_t s = stream ? (hipStream_t)stream : p->stream;
+    int rc = reserve_alias(*p, s);
+    if (!rc) rc = exec_plan(*p, direction, dst, src, s);
     if (rc == AFFT_OK) clear_error();
     return rc;
 }
@@ -730,7 +732,7 @@ int afft_plan_describe(afft_plan p, char* buf, int cap) {
 int64_t afft_plan_workspace_bytes(afft_plan p) {
     if (!p) return 0;
     int64_t t = 0;
-    for (int i = 0; i < NTMP; ++i) t += (int64_t)p->tmp_bytes[i];
+    for (int i = 0; i < NTMP; ++i) t += (int64_t)buffer_bytes(*p, i);
     return t;
 }
 

@@ -181,15 +181,22 @@ int afft_plan_inverse(afft_plan p, void* dst, int64_t dst_len, const void* src, 
  * and returns without synchronising.  A plan with workspace that is enqueued
  * on a different stream than its previous execution makes the new stream
  * wait for that execution first (outside stream capture), so executions of
- * one plan never overlap on its workspace; clones overlap freely. */
+ * one plan never overlap on its workspace; clones overlap freely.
+ * dst may be src.  Where dst overlaps src, some one-launch plans (real rows,
+ * rows with a prime factor above 7, long power-of-two columns) read a copy of
+ * the input unless every output lies exactly over its own input.  The first
+ * execution outside stream capture allocates the plan's workspace, the copy's
+ * buffer included, so later ones may be captured (complex rows whose copy
+ * exceeds 128 MiB allocate it in the first overlapping call instead). */
 int afft_plan_exec_device(afft_plan p, int direction, void* dst_dev, const void* src_dev, void* stream);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory while they execute (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): afft_plan_exec_device with the
  * plan's scratch taken from one static device array per GPU of
  * afft_noalloc_scratch_bytes() bytes (64 MiB) instead of memory the plan
- * allocates on its first execution.  Same kernels, same results.  A plan
- * whose workspace exceeds the array fails with ErrInvalidLength before
+ * allocates on its first execution.  Same kernels, same results.  A call
+ * whose workspace (that of its own buffers: see afft_plan_exec_device on
+ * overlapping ones) exceeds the array fails with ErrInvalidLength before
  * anything is enqueued.  All calls on one GPU share the array: calls that
  * overlap in time on one GPU race on it (order them on one stream). */
 int afft_plan_exec_device_noalloc(afft_plan p, int direction, void* dst_dev, const void* src_dev, void* stream);
@@ -211,7 +218,8 @@ int afft_plan_exec_buffers(afft_plan p, int direction, afft_buffer dst, afft_buf
 int afft_plan_synchronize(afft_plan p);
 /* Algorithm string recorded in wisdom (cf. Plan.Algorithm, plan.go:157). */
 int afft_plan_describe(afft_plan p, char* buf, int cap);
-/* Bytes of device workspace the plan holds. */
+/* Bytes of device workspace of the plan, the copy for overlapping buffers
+ * included; fixed at creation. */
 int64_t afft_plan_workspace_bytes(afft_plan p);
 int afft_plan_destroy(afft_plan p);           /* PlanImpl.Close */
 
