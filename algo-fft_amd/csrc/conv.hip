@@ -189,13 +189,14 @@ static void set_short(afft_conv_s& c) {
     if (c.short_lds <= 65536) c.short_fn = (const void*)&k_conv_short<T, REAL>;
 }
 
-// Direct sums up to as many taps as they are the faster form and no less
-// accurate than the transforms.  16.4 M points, transforms -> direct: float32 rows of
-// 1000 with 33 taps 0.080 -> 0.035 ms (error against 64 bits 2.0e-7 -> 1.0e-7), 64
-// 0.088 -> 0.047, 96 0.085 -> 0.061 (2.0e-7 -> 1.8e-7), 128 0.075 -> 0.079; complex64 rows of
-// 200 with 24 0.131 -> 0.087, of 1000 with 33 0.146 -> 0.088 (1.9e-7 -> 1.4e-7), 64 0.133
-// -> 0.135.  Rows whose transforms are launches of their own: complex64 of 100,000 with 64
-// 0.589 -> 0.117 (3.1e-7 -> 2.1e-7), complex128 of 16,000 with 128 0.468 -> 0.174.
+// Direct sums up to as many taps as they are the faster form; their error is
+// below the transforms' (kshort.hpp).  2^23 points (2^22 in double), transforms (at
+// one tap more) against direct sums: float32 rows of 1000 with 96 taps 45.8 us
+// against 32.6, of 200 35.1 against 39.2; float64 48.5 against 31.2 and 36.2
+// against 35.1; complex64 rows of 1000 with 48 68.7 against 64.3, of 5000 144
+// against 59; complex128 76.3 against 56.4 and 151 against 51.  Rows whose transforms are
+// launches of their own, 60 of 100,000 with 128: complex64 223 against 90,
+// complex128 377 against 157.
 static void prepare_short(afft_conv_s& c) {
     const bool real = c.mode == AFFT_CONV_REAL;
     const int64_t taps = std::min(c.na, c.nb);

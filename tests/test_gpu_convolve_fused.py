@@ -100,3 +100,32 @@ def test_short_sides(ctx, na, nb, batch, mode, prec):
     tol = c64_tol(na + nb) if prec == A.COMPLEX64 else C128_TOL
     assert np.all(got[-5:] == 7)
     assert rel_l2(got[:-5].reshape(batch, -1), _ref(a, b, mode)) <= tol
+
+
+# the direct form's rounding: a box filter over constant rows, where every
+# partial sum rounds alike.  With nonnegative terms each output is off by at most
+# one unit roundoff per addition on the way to it: 4 products of a side in
+# turn (2 taps' worth of either part for complex rows), the pair of them, 4 such
+# blocks, the groups of these.
+@pytest.mark.parametrize("taps,na", [(4, 100), (8, 200), (33, 1000), (48, 1000), (96, 1000), (128, 40000)])
+@pytest.mark.parametrize("mode", [A.CONV_LINEAR, A.CONV_REAL])
+@pytest.mark.parametrize("prec", [A.COMPLEX64, A.COMPLEX128])
+def test_box_filter_over_constant_rows(ctx, taps, na, mode, prec):
+    real = mode == A.CONV_REAL
+    if taps > 48 and not real and na < 16384:
+        pytest.skip("taken by the transforms")
+    half = 4 if real else 2   # taps summed in turn
+    depth = (min(taps, half) + (taps > half) + min(-(-taps // (2 * half)), 4) - 1 + -(-taps // (8 * half)) - 1) * (1 if real else 2)
+    u = 2.0 ** -24 if prec == A.COMPLEX64 else 2.0 ** -53
+    rdt = np.float32 if prec == A.COMPLEX64 else np.float64
+    dt = rdt if real else (np.complex64 if prec == A.COMPLEX64 else np.complex128)
+    c = np.concatenate([np.linspace(1, 2, 60), [1.9296482, 1.8442211, 1.0653267]]).astype(rdt)
+    h = rdt(1.0 / taps)
+    a = np.repeat(c[:, None], na, axis=1).astype(dt)
+    b = np.full((len(c), taps), h, dt)
+    ta, tb = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    out = torch.empty((len(c), na + taps - 1), dtype=ta.dtype, device="cuda")
+    _run(ctx, prec, mode, na, taps, len(c), out, ta, tb)
+    got = out.cpu().numpy()[:, taps - 1:na].real
+    ref = (c.astype(np.longdouble) * np.longdouble(h) * taps)[:, None]
+    assert float(np.max(np.abs(got - ref) / ref)) <= depth * u
