@@ -960,7 +960,8 @@ static int emit_gen_fourstep(Plan& p, int di, const AxisJob& j, std::string& alg
     } else if ((rc = mix_args(p, n2, MIX_TROWS, n1, cc, gb, mb))) {
         return rc;
     }
-    if ((rc = split_twiddles(p, prec, j.n, &ga.k.tw4_shift, &ga.k.tw4_lo, &ga.k.tw4_hi))) return rc;
+    // k_mix reads its four-step tables in double for either precision
+    if ((rc = split_twiddles(p, ka ? prec : 1, j.n, &ga.k.tw4_shift, &ga.k.tw4_lo, &ga.k.tw4_hi))) return rc;
     const void* fa = ka ? ka->fn : mix_kernel(prec, VAR_4A, dir);
     const void* fb = kb ? kb->fn : mix_kernel(prec, VAR_4B, dir);
     if ((!ka && (rc = prep_dynamic_lds(fa, ma.lds))) || (!kb && (rc = prep_dynamic_lds(fb, mb.lds)))) return rc;
