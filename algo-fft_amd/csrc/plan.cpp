@@ -613,7 +613,22 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
     const double conf = lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012;
     const int minp = mix_min_passes(n, MIX_MAXPASS);
-    if (minp > MIX_MAXPASS) return false;
+    if (minp > MIX_MAXPASS || (lay == MIX_TROWS ? n | 1 : n + pad) * es > 163840) return false;
+    // Radices that the largest block holds, and the numbers of passes (bit p:
+    // p passes) in which they make up a rest of n: orders that no block size fits
+    // are never listed.  (Listing them took up to 15 ms a length; 300 rows of a
+    // rough length look at many: plans of 9174 complex64 points 90 -> 2.6 ms, of 10007
+    // 41 -> 2.7.)
+    auto usable = [&](int q) { return n % q == 0 && (n / q + mix_mb(q) - 1) / mix_mb(q) <= maxth; };
+    std::map<int64_t, unsigned> reach{{1, 1u}};
+    auto passes_of = [&](auto&& self, int64_t rest) -> unsigned {
+        const auto hit = reach.find(rest);
+        if (hit != reach.end()) return hit->second;
+        unsigned r = 0;
+        for (int q : kMixRadices)
+            if (rest % q == 0 && usable(q)) r |= self(self, rest / q) << 1;
+        return reach[rest] = r;
+    };
     std::vector<std::pair<double, MixShape>> top;   // sorted, the cheapest few
     constexpr size_t KEEP = 12;
     std::vector<int> rad;
@@ -669,9 +684,9 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
             consider();
             return;
         }
-        if ((int)rad.size() == passes) return;
+        const int left = passes - (int)rad.size();
         for (int q : kMixRadices) {
-            if (rest % q) continue;
+            if (rest % q || !usable(q) || !(passes_of(passes_of, rest / q) >> (left - 1) & 1)) continue;
             rad.push_back(q);
             self(self, rest / q, passes);
             rad.pop_back();
@@ -679,7 +694,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
     };
     // more passes only where no schedule of the fewest fits the block size
     for (int passes = minp; passes <= MIX_MAXPASS && (passes <= minp + 1 || top.empty()); ++passes)
-        extend(extend, n, passes);
+        if (passes_of(passes_of, n) >> passes & 1) extend(extend, n, passes);
     if (top.empty()) return false;
     double best = 1e300;
     for (auto& t : top) {
@@ -745,15 +760,21 @@ MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw) {
 // images 814 -> 540, of 1200 x 1500 complex128 grids 542 -> 286.
 struct MixCache {
     std::map<std::tuple<int64_t, int, int64_t, int64_t, int>, std::pair<MixArgs, MixShape>> known;
+    std::map<std::tuple<int64_t, int64_t, int64_t>, int64_t> padded;   // blue_smooth_length by n, count, slices
 };
+
+static MixCache& mix_cache(Plan& p) {
+    if (!p.mix_cache) p.mix_cache = std::make_shared<MixCache>();
+    return *p.mix_cache;
+}
 
 // Kernel arguments of a launch shape and their twiddle tables, in a cleared a.
 static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t slices, MixArgs& a, MixShape& m,
                     int pad = 0) {
-    if (!p.mix_cache) p.mix_cache = std::make_shared<MixCache>();
+    MixCache& cache = mix_cache(p);
     const auto key = std::make_tuple(n, (int)lay, count, slices, pad);
-    const auto hit = p.mix_cache->known.find(key);
-    if (hit != p.mix_cache->known.end()) {
+    const auto hit = cache.known.find(key);
+    if (hit != cache.known.end()) {
         std::tie(a, m) = hit->second;
         return AFFT_OK;
     }
@@ -778,7 +799,7 @@ static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t sl
     } else {
         rc = upload_table(p, tw.data(), tw.size() * 8, &a.k.tw);
     }
-    if (rc == AFFT_OK) p.mix_cache->known.emplace(key, std::make_pair(a, m));
+    if (rc == AFFT_OK) cache.known.emplace(key, std::make_pair(a, m));
     return rc;
 }
 
@@ -1412,7 +1433,10 @@ static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) 
             is_prime(n) && !smooth_schedule(n - 1).empty() &&
             mix_shape(n - 1, prec, MIX_ROWS, j.count, j.slices, ms, nullptr, 1))
             return emit_mix_blue(p, di, j, n - 1, true, algo);
-        if (const int64_t sm = blue_smooth_length(n, m, prec, j.count, j.slices))
+        auto& padded = mix_cache(p).padded;
+        const auto key = std::make_tuple(n, j.count, j.slices);
+        if (!padded.count(key)) padded[key] = blue_smooth_length(n, m, prec, j.count, j.slices);
+        if (const int64_t sm = padded[key])
             return emit_mix_blue(p, di, j, sm, false, algo);
     }
     if (m <= max_single_pass(prec)) {
