@@ -562,15 +562,29 @@ static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout 
 // of 512 MiB in both precisions: the pick is on average 2.4 % (rows), 4.4 %
 // (columns) and 6.6 % (transposing rows) slower than the best one, 25 % at
 // worst.
-static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total) {
+//
+// few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few).  These are over
+// before their blocks have to share the CUs: a block's own time decides, the
+// passes and the points that a thread takes in turn, not the occupancy and the
+// conflicts.  On every shape of 360 row cases, 128 Rader rows and 184 column
+// cases of up to 2^20 points (10 to 8000 a transform, both precisions) the picks are 2.9, 2.7
+// and 3.5 % slower than the best in the mean, 21, 29 and 20 % at worst; by the
+// other terms alone 7.7, 6.2 and 28 %, 62, 33 and 125 % (complex64 columns 625 x 33 11.4 ->
+// 5.4 us, 1225 x 500 11.2 -> 8.3; 1245 rows of 421 points 11.2 -> 8.6).
+static double mix_few(int64_t n, int64_t count, int64_t slices, int prec) {
+    return std::clamp(23.0 - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
+}
+
+static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total, double few) {
     const int es = prec ? 16 : 8, wps = prec ? 3 : 5, waves = m.threads / 64;
     const int by_waves = waves <= 8 ? wps * 4 / waves : wps / ((waves + 3) / 4);
     const int blocks = std::max(1, std::min({(int)(163840 / std::max(m.lds, 1)), by_waves, 32}));
     const double P = (double)m.rad.size(), inv = 1.0 / blocks, one = blocks == 1 ? 1.0 : 0.0, th = m.threads / 1024.0;
-    double work = -P;
+    double work = -P, serial = 0;
     for (int q : m.rad) {
-        const int64_t nr = n / q;
-        work += (double)m.threads / m.g * ((nr + m.tpt - 1) / m.tpt) * q / n;
+        const int64_t rounds = (n / q + m.tpt - 1) / m.tpt;
+        work += (double)m.threads / m.g * rounds * q / n;
+        serial += (double)rounds * q;
     }
     const double seg = m.g * es, seg128 = std::max(0.0, 128 / seg - 1), seg64 = seg < 64 ? 1.0 : 0.0;
     const double rl = 128.0 / (std::min<int64_t>(m.tpt, n / m.rad.front()) * es);
@@ -579,10 +593,12 @@ static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, in
     const double idle = blocks_total < 256 ? std::log2(256.0 / blocks_total) : 0.0;
     switch (lay) {
     case MIX_ROWS:
-        return P + 0.105 * work + 0.538 * inv + 0.113 * one + 0.056 * rl + 0.035 * rs + 0.029 * rl * rl +
-               0.037 * rs * rs - 0.433 * th + idle;
+        return P + few * (serial / 64 + 0.1 * th) +
+               (1 - few) * (idle + 0.105 * work + 0.538 * inv + 0.113 * one + 0.056 * rl + 0.035 * rs + 0.029 * rl * rl +
+                            0.037 * rs * rs - 0.433 * th);
     case MIX_COLS:
-        return P + 0.546 * work + 1.647 * inv + 3.575 * one + 1.155 * seg128 + 1.173 * seg64 - 1.645 * th + idle;
+        return P + few * (serial / 64 + 0.4 * th + 0.5 * idle + 0.023 * (seg128 + seg64)) +
+               (1 - few) * (idle + 0.546 * work + 1.647 * inv + 3.575 * one + 1.155 * seg128 + 1.173 * seg64 - 1.645 * th);
     default:
         return P + 0.054 * work + 1.81 * inv + 0.05 * one + 0.886 * seg128 + 0.106 * seg64 + 0.205 * rl -
                0.0092 * m.rad.front() - 0.143 * th + idle;
@@ -605,13 +621,19 @@ static int mix_min_passes(int64_t n, int most) {
 // passes, and with one more where they are within a factor 1.7 of each
 // other, times every thread count that gives some pass whole butterflies,
 // times the group sizes; the bank conflicts rank the cheapest of them.
+// Lengths of one pass try any two: from memory such rows are a thread's each, half of them
+// a line (2^23 complex64 points in rows of 10, 14 and 18: one pass 46, 47, 54 us, two
+// 30 to 33).  Rows with a slot to spare (pad) come through LDS: below 12 points
+// one pass is theirs, from 16 on two (16000 complex64 rows of 11 points by Rader's 10
+// 5.0 us, 5 x 2 5.6; of 17 by 16 6.3, 4 x 4 5.7; of 19 by 18 7.0, 6 x 3 6.2).
 // Radices up to 10 hold 16 points per thread, so at most n/16 threads (the
 // largest block at the largest length) always fit.
 // pad: LDS slots of a row beyond its n points.
 static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out,
                       double* cost = nullptr, int pad = 0) {
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
-    const double conf = lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012;
+    const double few = lay == MIX_TROWS ? 0.0 : mix_few(n, count, slices, prec);
+    const double conf = (1 - few) * (lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012);
     const int minp = mix_min_passes(n, MIX_MAXPASS);
     if (minp > MIX_MAXPASS || (lay == MIX_TROWS ? n | 1 : n + pad) * es > 163840) return false;
     // Radices that the largest block holds, and the numbers of passes (bit p:
@@ -665,7 +687,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
                 m.lds = (int)lds;
                 m.threads = (m.g * m.tpt + 63) / 64 * 64;
                 m.rad = rad;
-                const double c = mix_cost(m, n, prec, lay, std::max<int64_t>(1, (count + m.g - 1) / m.g * slices));
+                const double c = mix_cost(m, n, prec, lay, std::max<int64_t>(1, (count + m.g - 1) / m.g * slices), few);
                 if (top.size() == KEEP && c >= top.back().first) continue;
                 auto it = top.begin();
                 while (it != top.end() && it->first <= c) ++it;
@@ -679,7 +701,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
             if ((int)rad.size() != passes) return;
             if (passes == minp + 1 && !top.empty()) {
                 const auto mm = std::minmax_element(rad.begin(), rad.end());
-                if (*mm.second * 10 > *mm.first * 17) return;
+                if (minp == 1 ? pad && n < 12 : *mm.second * 10 > *mm.first * 17) return;
             }
             consider();
             return;
@@ -693,7 +715,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
         }
     };
     // more passes only where no schedule of the fewest fits the block size
-    for (int passes = minp; passes <= MIX_MAXPASS && (passes <= minp + 1 || top.empty()); ++passes)
+    for (int passes = pad && n >= 16 ? std::max(2, minp) : minp; passes <= MIX_MAXPASS && (passes <= minp + 1 || top.empty()); ++passes)
         if (passes_of(passes_of, n) >> passes & 1) extend(extend, n, passes);
     if (top.empty()) return false;
     double best = 1e300;
@@ -1398,6 +1420,10 @@ static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count,
         double cost;
         if (smooth_schedule(c).empty() || !mix_shape(c, prec, MIX_ROWS, count, slices, ms, &cost)) continue;
         ++seen;
+        // 256 complex64 points are two passes of the compile-time kernel: 2^23 points of
+        // rows of 86 53.7 us, 89.6 padded to 175 = 7 x 5 x 5; of 79 54.3, 55.5 padded to
+        // 160 = 10 x 16, whose LDS rows conflict
+        if (!prec && m == 256 && (ms.rad.size() > 2 || std::count(ms.rad.begin(), ms.rad.end(), 16))) continue;
         if (m > max_single_pass(prec) && ms.rad.size() > 4 && count * slices < 256) continue;
         if ((cost - 1) * (double)c < least) {
             least = (cost - 1) * (double)c;
