@@ -310,8 +310,16 @@ static int emit_single(Plan& p, int di, const AxisJob& j, std::string& algo) {
     a.in_bd = in_bd;
     a.out_bd = out_bd;
     a.scale = j.scale;
-    a.xcd = var == VAR_COL && xcd_order(j.in_nd * es, j.out_nd * es);
     const int64_t gx = (count + k->tpb - 1) / k->tpb;
+    // Column groups that start and end on lines, or have none beside them, share
+    // nothing.  There XCD order pays from 64 MiB on; in what the caches hold it takes a block
+    // away from the XCD whose L2 the pass before has filled (XCD -> plain order: complex128
+    // 8 x 32 x 4096 18.5 -> 13.3 us, 8 x 8 x 128 x 128 30.1 -> 24.4, complex64 64 x 16 x 1024 13.9 -> 11.2,
+    // 64 x 64 x 1024 28.1 -> 25.3; the four-step's columns want it at any size: 65536 x 16
+    // 13.2 against 15.9).
+    const bool apart = gx < 2 || (j.in_nd * es % 128 == 0 && j.out_nd * es % 128 == 0);
+    a.xcd = var == VAR_COL && xcd_order(j.in_nd * es, j.out_nd * es) &&
+            (!apart || j.n * count * slices * es >= int64_t(64) << 20);
     Step s = make_step(k, a, gx, 1, var == VAR_ROW ? "row" : "col", gx * slices);
     // rows whose threads cover less than a line at a time: no streaming, which
     // would take the partial lines to memory one by one (complex64, 512 MiB: 8
@@ -1705,7 +1713,11 @@ static int emit_axis_direct(Plan& p, int di, const AxisJob& j, std::string& algo
     // fewer are one thread's either way (complex64 8 points 0.350 against
     // 0.388), and at 1 KiB the compile-time kernel wins on cached batches
     // (complex64 128 points, 32 MiB: 11.7 against 14.2 us).
-    if (is_pow2(j.n) && rows && j.n >= 16 && j.n * (prec ? 16 : 8) <= 512 &&
+    // Rows of 64 complex64 points before other axes stay there beyond 16 MiB, where the
+    // next pass finds more of its input in its L2 (32 MiB: 16 x 64 x 4096 29.0 -> 25.5 us,
+    // 64 x 64 x 1024 25.3 -> 24.3, 64 x 64 x 64 x 16 37.7 -> 34.9; 8 MiB and 128 MiB even).
+    const bool inner64 = p.desc.rank > 1 && !prec && j.n == 64 && j.count * j.slices > 32768;
+    if (is_pow2(j.n) && rows && j.n >= 16 && j.n * (prec ? 16 : 8) <= 512 && !inner64 &&
         !(p.desc.flags & AFFT_FLAG_MFMA))
         return emit_gen_single(p, di, j, algo);
     // Long power-of-two columns, many side by side: 32 KiB of column and more
