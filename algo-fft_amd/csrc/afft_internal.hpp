@@ -156,6 +156,17 @@ int prep_dynamic_lds(const void* fn, int lds);
 // thread) in LDS rows of the given pitch, every pass in place: the fewest
 // passes, then the least idle lanes and bank conflicts.
 std::vector<int> mix_lds_schedule(int64_t n, int prec, int tpt, int pitch);
+// Fewest passes of the runtime radices for a 7-smooth n.
+int mix_passes(int64_t n);
+// How `count * slices` rows of a length outside the radices run: Rader's form on
+// m = n - 1 points, or Bluestein's padded to a 7-smooth m or the power of two.
+enum { BLUE_ROUTE_POW2, BLUE_ROUTE_SMOOTH, BLUE_ROUTE_RADER };
+struct BlueRoute {
+    int kind = BLUE_ROUTE_POW2;
+    int64_t m = 0;
+    int launches = 1;
+};
+BlueRoute blue_route(int64_t n, int prec, int64_t count, int64_t slices, bool refchirp, bool rader);
 // Appends the twiddles of a pass (mix_twiddle's entries) to tw and returns it.
 struct MixPass;
 MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw);

@@ -625,6 +625,8 @@ static int mix_min_passes(int64_t n, int most) {
     return best;
 }
 
+int mix_passes(int64_t n) { return mix_min_passes(n, MIX_MAXPASS); }
+
 // Launch shape of n 7-smooth points: every order of radices with the fewest
 // passes, and with one more where they are within a factor 1.7 of each
 // other, times every thread count that gives some pass whole butterflies,
@@ -790,7 +792,7 @@ MixPass mix_pass_tables(int64_t n, int R, int64_t ns, std::vector<double>& tw) {
 // images 814 -> 540, of 1200 x 1500 complex128 grids 542 -> 286.
 struct MixCache {
     std::map<std::tuple<int64_t, int, int64_t, int64_t, int>, std::pair<MixArgs, MixShape>> known;
-    std::map<std::tuple<int64_t, int64_t, int64_t>, int64_t> padded;   // blue_smooth_length by n, count, slices
+    std::map<std::tuple<int64_t, int64_t, int64_t>, BlueRoute> routes;   // by n, count, slices
 };
 
 static MixCache& mix_cache(Plan& p) {
@@ -1441,38 +1443,45 @@ static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count,
     return best;
 }
 
+// Plans with the reference's chirp (refchirp) stay on its padded lengths.  Rader's form
+// halves the points of the convolution: primes of 2^24 complex64 points, from
+// the padded form: 31 points 0.112 -> 0.106 ms, 257 0.215 -> 0.095, 1009 0.138
+// -> 0.091, 4051 0.24 -> 0.126, 8101 0.22 -> 0.144; 2^23 complex128: 61 0.115 -> 0.085,
+// 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.  A few rows are through the
+// compile-time kernel sooner where m is 2048 or 4096 (complex64 1009: 64 rows
+// 8.9 against 11.4 us, 1024 11.3 against 11.8, 2048 17.7 against 16.6; 2017: 512
+// rows 11.5 against 14.5, 1024 18.2 against 17.6) or very short (17: 64
+// rows 5.6 against 5.7).
+// Where the power of two is beyond LDS a row is one block's, the chain spreads
+// it over many: one launch from 64 rows on (complex128 4099 points, chain -> one
+// launch: 1 row 19.5 -> 25.7 us, 32 27.5 -> 26.3, 64 31.3 -> 26.7, 256 67 -> 33;
+// complex64 18433: 1 row 19.9 -> 41.5, 64 43.4 -> 42.8, 256 122 -> 52).
+BlueRoute blue_route(int64_t n, int prec, int64_t count, int64_t slices, bool refchirp, bool rader) {
+    const int64_t m = next_pow2(2 * n - 1);
+    if (!refchirp && (m <= max_single_pass(prec) || count * slices >= 64)) {
+        MixShape ms;
+        const int64_t fewest = m <= 128 ? 1 << 15 : m <= 1024 || m > 4096 ? 0 : 1 << 22;
+        if (rader && count * slices * m >= fewest && n < 65536 && is_prime(n) && !smooth_schedule(n - 1).empty() &&
+            mix_shape(n - 1, prec, MIX_ROWS, count, slices, ms, nullptr, 1))
+            return {BLUE_ROUTE_RADER, n - 1, 1};
+        if (const int64_t sm = blue_smooth_length(n, m, prec, count, slices)) return {BLUE_ROUTE_SMOOTH, sm, 1};
+    }
+    return {BLUE_ROUTE_POW2, m, m <= max_single_pass(prec) ? 1 : 3};
+}
+
 static int emit_bluestein(Plan& p, int di, const AxisJob& j, std::string& algo) {
     const int prec = p.desc.precision;
     const int dir = di ? 1 : -1;
     const int es = prec ? 16 : 8;
     if (j.in_nd != 1 || j.out_nd != 1) return set_error(AFFT_ERR_NOT_IMPLEMENTED, "Bluestein needs unit stride");
     const int64_t n = j.n, m = next_pow2(2 * n - 1);
-    // Plans with the reference's chirp stay on its padded lengths.  Rader's form
-    // halves the points of the convolution: primes of 2^24 complex64 points, from
-    // the padded form: 31 points 0.112 -> 0.106 ms, 257 0.215 -> 0.095, 1009 0.138
-    // -> 0.091, 4051 0.24 -> 0.126, 8101 0.22 -> 0.144; 2^23 complex128: 61 0.115 -> 0.085,
-    // 1009 0.132 -> 0.092, 8101 0.30 -> 0.175.  A few rows are through the
-    // compile-time kernel sooner where m is 2048 or 4096 (complex64 1009: 64 rows
-    // 8.9 against 11.4 us, 1024 11.3 against 11.8, 2048 17.7 against 16.6; 2017: 512
-    // rows 11.5 against 14.5, 1024 18.2 against 17.6) or very short (17: 64
-    // rows 5.6 against 5.7).
-    // Where the power of two is beyond LDS a row is one block's, the chain spreads
-    // it over many: one launch from 64 rows on (complex128 4099 points, chain -> one
-    // launch: 1 row 19.5 -> 25.7 us, 32 27.5 -> 26.3, 64 31.3 -> 26.7, 256 67 -> 33;
-    // complex64 18433: 1 row 19.9 -> 41.5, 64 43.4 -> 42.8, 256 122 -> 52).
-    if (!(p.desc.flags & AFFT_FLAG_REF_CHIRP) && (m <= max_single_pass(prec) || j.count * j.slices >= 64)) {
-        MixShape ms;
-        const int64_t fewest = m <= 128 ? 1 << 15 : m <= 1024 || m > 4096 ? 0 : 1 << 22;
-        if (p.desc.strategy != AFFT_STRATEGY_BLUESTEIN && j.count * j.slices * m >= fewest && n < 65536 &&
-            is_prime(n) && !smooth_schedule(n - 1).empty() &&
-            mix_shape(n - 1, prec, MIX_ROWS, j.count, j.slices, ms, nullptr, 1))
-            return emit_mix_blue(p, di, j, n - 1, true, algo);
-        auto& padded = mix_cache(p).padded;
-        const auto key = std::make_tuple(n, j.count, j.slices);
-        if (!padded.count(key)) padded[key] = blue_smooth_length(n, m, prec, j.count, j.slices);
-        if (const int64_t sm = padded[key])
-            return emit_mix_blue(p, di, j, sm, false, algo);
-    }
+    auto& routes = mix_cache(p).routes;
+    const auto key = std::make_tuple(n, j.count, j.slices);
+    if (!routes.count(key))
+        routes[key] = blue_route(n, prec, j.count, j.slices, p.desc.flags & AFFT_FLAG_REF_CHIRP,
+                                 p.desc.strategy != AFFT_STRATEGY_BLUESTEIN);
+    const BlueRoute route = routes[key];
+    if (route.kind != BLUE_ROUTE_POW2) return emit_mix_blue(p, di, j, route.m, route.kind == BLUE_ROUTE_RADER, algo);
     if (m <= max_single_pass(prec)) {
         BlueTables bt;
         int rc = blue_tables(p, n, m, 0.0, bt);

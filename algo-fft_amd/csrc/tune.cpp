@@ -120,24 +120,26 @@ void plan_features(const afft_plan_desc& d, const Candidate& c, float* f) {
     for (int i = 0; i < 4; ++i)
         while (m % q[i] == 0) { m /= q[i]; ++e[i]; }
     const bool smooth = m == 1;
-    // executed FFT length: the Bluestein padding for a Bluestein candidate
-    // (also for smooth n), else n
+    // executed FFT length: that of the convolution for a Bluestein candidate
+    // (also for smooth n; rough lengths may take Rader's form), else n
     const bool blue = c.strategy == AFFT_STRATEGY_BLUESTEIN || (c.strategy == AFFT_STRATEGY_AUTO && !smooth);
-    const int64_t M = blue ? [&] { int64_t v = 1; while (v < 2 * n - 1) v <<= 1; return v; }() : n;
+    const BlueRoute route = blue ? blue_route(n, prec, b, 1, d.flags & AFFT_FLAG_REF_CHIRP, !smooth) : BlueRoute{};
+    const int64_t M = blue ? route.m : n;
     const int64_t stride = d.istride > 1 ? d.istride : 1;
     int64_t n1 = c.split, n2 = c.split ? n / c.split : 0;
     if (c.strategy == AFFT_STRATEGY_SIXSTEP && !n1) { n1 = 1LL << (ilog2i(n) / 2); n2 = n / n1; }
     const double es = prec ? 16.0 : 8.0;
     int launches = 1;
     if (c.strategy == AFFT_STRATEGY_SIXSTEP) launches = 2;
-    if (c.strategy == AFFT_STRATEGY_BLUESTEIN) launches = M <= max_single_pass(prec) ? 1 : 4;
-    // radix passes of a length and how many of them are odd (3, 5, 7)
+    if (blue) launches = route.launches;
+    // radix passes of a length (powers of two on the compile-time kernels, else
+    // the runtime radices) and its odd prime factors
     auto passes = [](int64_t len, int* odd) {
         *odd = 0;
         if (len < 2) return 0;
         std::vector<int> r = smooth_schedule(len);
         for (int x : r) *odd += (x & 1);
-        return (int)r.size();
+        return is_pow2(len) ? (int)r.size() : mix_passes(len);
     };
     int odd_n = 0, odd1 = 0, odd2 = 0;
     const int pn = passes(M, &odd_n);
@@ -265,6 +267,8 @@ int afft_tune_plan(afft_context ctx, const afft_plan_desc* d, int warmup, int it
         afft_plan_desc q = *d;
         q.strategy = cand[i].strategy;
         q.split = cand[i].split;
+        // a rough length's only candidate stands for what plans of it run
+        if (smooth_schedule(d->dims[0]).empty()) q.strategy = AFFT_STRATEGY_AUTO;
         double t = -1;
         if (time_desc(ctx, q, warmup, iters, &t) != AFFT_OK) t = -1;
         if (times && (int)i < cap) times[i] = t;

@@ -203,3 +203,23 @@ def test_cost_model_regret_on_freshly_timed_shapes(ctx):
           f"; mean {mean_model:.4f}")
     assert all(r[0] <= 0.10 for r in res)
     assert mean_model <= r_heur
+
+
+def test_tuner_times_what_plans_of_a_rough_length_run(ctx):
+    """The only candidate of a prime is timed on the route of its plans (Rader's form
+    here: 50 us, the padded form that the forced strategy takes 70)."""
+    import ctypes
+    sh = {"n": 1009, "batch": 8192, "precision": A.COMPLEX64, "stride": 1}
+
+    def time_of(strategy):
+        ms = ctypes.c_double()
+        d = planner.desc_for(sh, strategy)
+        A.check(A.lib().afft_tune_time(ctx.h, ctypes.byref(d), 20, 50, ctypes.byref(ms)))
+        return ms.value
+
+    times = (ctypes.c_double * 1)()
+    d = planner.desc_for(sh)
+    with A.Context(0) as own:   # the winner's wisdom stays out of the shared context
+        A.check(A.lib().afft_tune_plan(own.h, ctypes.byref(d), 20, 50, None, None, None, times, 1))
+    auto, forced = time_of(A.STRATEGY_AUTO), time_of(A.STRATEGY_BLUESTEIN)
+    assert abs(times[0] - auto) < abs(times[0] - forced), (times[0], auto, forced)

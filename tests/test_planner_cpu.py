@@ -72,3 +72,16 @@ def test_default_smooth_fourstep_split_is_a_candidate():
             assert n % s == 0
             c = planner.candidates({"n": n, "batch": 4, "precision": prec, "stride": 1})
             assert (A.STRATEGY_SIXSTEP, s) in c, (n, prec, s, c)
+
+
+def test_features_follow_the_executed_convolution():
+    # f[11] log2 of the executed length, f[23] launches, f[28] radix passes
+    def f(n, batch, prec=A.COMPLEX64, strategy=A.STRATEGY_BLUESTEIN):
+        return planner.features({"n": n, "batch": batch, "precision": prec, "stride": 1}, strategy, 0)
+    assert f(1009, 8192)[11] == np.float32(math.log2(1008))      # Rader's form
+    assert f(1009, 64)[11] == 11                                 # few rows: 2048
+    assert f(2053, 8172)[11] == np.float32(math.log2(4200))      # padded to 4200 = 20 x 15 x 14
+    chain = f(100003, 4)
+    assert chain[11] == 18 and chain[23] == 3                    # 2^18 in three passes
+    assert f(1009, 8192, strategy=A.STRATEGY_AUTO)[23] == 1
+    assert f(3000, 16, strategy=A.STRATEGY_MIXED)[28] == 3       # 15 x 20 x 10
