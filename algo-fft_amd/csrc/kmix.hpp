@@ -41,9 +41,9 @@ struct MixArgs {
     int pitch;            // LDS row pitch (row layouts)
 };
 
-// Butterflies of radix R that a thread may hold in one pass: 14 to 21 points.
-// At least 16 points for every radix from 2 to 10 but 7 (21), so a schedule
-// of at most N/16 threads a transform always exists.
+// Butterflies of radix R that a thread may hold in one pass: 12 to 21 points,
+// at least 16 for every radix from 2 to 10, so a schedule of at most N/16
+// threads a transform always exists.
 __host__ __device__ constexpr int mix_mb(int R) {
     return R >= 12 ? 1 : R >= 8 ? 2 : R >= 6 ? 3 : R == 5 ? 4 : R == 4 ? 5 : R == 3 ? 6 : 8;
 }

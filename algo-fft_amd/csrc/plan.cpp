@@ -3,12 +3,23 @@
 //
 // Size routing (cf. the reference's planner.go:43-78, which picks codelets,
 // Stockham, six-step or Bluestein for a CPU):
-//   power of two <= LDS capacity (16384 c64 / 8192 c128)  one LDS pass
+//   power of two <= LDS capacity (16384 c64 / 8192 c128)  one LDS pass; rows of 16 points to
+//                                                         512 bytes and many long columns
+//                                                         on the runtime radices
 //   power of two above it                                 four-step: column pass with
 //                                                         fused twiddle, then a row pass
 //                                                         whose store transposes
-//   2/3/5/7-smooth                                        runtime mixed-radix Stockham
-//   anything else                                         fused Bluestein chain
+//   2/3/5/7-smooth                                        runtime radices (k_mix): one pass
+//                                                         held in LDS, else four-step
+//   anything else (blue_route)                            one launch: Rader's form, or
+//                                                         Bluestein's padded to a smooth
+//                                                         length or a power of two; where
+//                                                         LDS does not hold it, or few
+//                                                         rows would leave the chip idle,
+//                                                         Bluestein's in three passes
+// How many transforms a plan has decides too: launch shapes, Rader or padded
+// form and planar exchanges follow it, so the last bits of a transform may
+// differ between plans of different batches (never between runs of one plan).
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -586,7 +597,9 @@ static double mix_few(int64_t n, int64_t count, int64_t slices, int prec) {
 static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total, double few) {
     const int es = prec ? 16 : 8, wps = prec ? 3 : 5, waves = m.threads / 64;
     const int by_waves = waves <= 8 ? wps * 4 / waves : wps / ((waves + 3) / 4);
-    const int blocks = std::max(1, std::min({(int)(163840 / std::max(m.lds, 1)), by_waves, 32}));
+    // blocks of exactly half a CU's LDS do not pair: complex128 columns of 640 points, 13107
+    // in blocks of 8 (80 KiB) 83 us, of 4 57; of 1280 points 80 and 62
+    const int blocks = std::max(1, std::min({(int)(163839 / std::max(m.lds, 1)), by_waves, 32}));
     const double P = (double)m.rad.size(), inv = 1.0 / blocks, one = blocks == 1 ? 1.0 : 0.0, th = m.threads / 1024.0;
     double work = -P, serial = 0;
     for (int q : m.rad) {

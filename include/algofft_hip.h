@@ -164,7 +164,9 @@ int afft_plan_create(afft_context ctx, int64_t n, int precision, const afft_plan
 /* Extended constructor: batch/stride (Plan.ForwardBatch, plan.go:504;
  * Plan.ForwardStrided, plan_strided.go:16), real (NewPlanReal32/64,
  * plan_real_constructors.go:8-43) and N-D (NewPlan2D/3D/ND, plan_2d.go:44,
- * plan_3d.go:42, plan_nd.go:43). */
+ * plan_3d.go:42, plan_nd.go:43).  Kernels and launch shapes follow the batch
+ * as well as the length: the last bits of a transform may differ between plans
+ * of different batches, never between executions of one plan. */
 int afft_plan_create_desc(afft_context ctx, const afft_plan_desc* desc, afft_plan* out);
 int64_t afft_plan_len(afft_plan p);           /* PlanImpl.Len: points of one transform */
 int afft_plan_precision(afft_plan p);         /* PlanImpl.Precision */

@@ -54,6 +54,12 @@ def test_few_columns(ctx, n, cols, prec, dt):
     _run(ctx, n, cols, prec, dt, columns=True)
 
 
+# many columns, blocks below half a CU's LDS
+@pytest.mark.parametrize("n,cols", [(320, 4099), (640, 4099), (1280, 2051)])
+def test_many_columns(ctx, n, cols):
+    _run(ctx, n, cols, A.COMPLEX128, torch.complex128, columns=True)
+
+
 # padded to 175 points in three passes these rows took 90 us where the two passes
 # of 256 take 54
 @pytest.mark.parametrize("n", [85, 86, 87, 88])
