@@ -949,15 +949,13 @@ static int emit_gen_single(Plan& p, int di, const AxisJob& j, std::string& algo)
 // kernel) or a runtime-radix length of 8 to 4096 points (the in-place
 // column kernel, at most 16 points per thread), with n1/sqrt(n) in
 // [0.2, 5].  A factor costs 3 on the compile-time kernel, else one per pass
-// plus one per radix-2 and a half per radix-4 pass; ties go to the more
-// balanced pair, then the smaller n1.  Fitted on 33 complex64 / complex128
-// lengths from 9000 to 10^6 with every such split timed on 512 MiB batches:
-// 5.4 % mean regret, 29 % at worst (5.8 % and 6.0 % on either half fitted
-// on the other), against 15.6 % and 71 % for the earlier rule (the
-// power-of-two part as the column
-// factor when 16..4096 points with the rest at most 2048, else the most
-// balanced divisors): complex64 18000 as 16 x 1125 took 0.99 ms against
-// 0.59 ms as 225 x 80, 30000 as 16 x 1875 1.06 against 0.62 ms.  Lengths
+// plus one per radix-2 and a half per radix-4 pass (of smooth_schedule's
+// radices); ties go to the more balanced pair, then the smaller n1.  Fitted on 33
+// complex64 / complex128 lengths from 9000 to 10^6 on kernels with one radix of {2, 3,
+// 4, 5, 7, 8, 16} a pass: 5.4 % mean regret there, against 15.6 % for the power-of-two
+// part as the column factor.  On the composite radices it is 7.7 % over 599
+// shapes of the tuning records, 79 % at worst (12042240 as 735 x 16384 0.238 ms, 3136 x 3840
+// 0.133); wisdom and the cost model pick among the timed splits.  Lengths
 // with no such pair take the most balanced divisors within the caps.
 int64_t gen_fourstep_split(int64_t n, int prec) {
     const int64_t cap = gen_cap(prec), rcap = std::min<int64_t>(cap, 4096);
