@@ -582,7 +582,8 @@ static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout 
 // (columns) and 6.6 % (transposing rows) slower than the best one, 25 % at
 // worst.
 //
-// few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few).  These are over
+// few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few; twice that for rows
+// through LDS, which compute longer on as much).  These are over
 // before their blocks have to share the CUs: a block's own time decides, the
 // passes and the points that a thread takes in turn, not the occupancy and the
 // conflicts.  On every shape of 360 row cases, 128 Rader rows and 184 column
@@ -590,11 +591,16 @@ static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout 
 // and 3.5 % slower than the best in the mean, 21, 29 and 20 % at worst; by the
 // other terms alone 7.7, 6.2 and 28 %, 62, 33 and 125 % (complex64 columns 625 x 33 11.4 ->
 // 5.4 us, 1225 x 500 11.2 -> 8.3; 1245 rows of 421 points 11.2 -> 8.6).
-static double mix_few(int64_t n, int64_t count, int64_t slices, int prec) {
-    return std::clamp(23.0 - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
+static double mix_few(int64_t n, int64_t count, int64_t slices, int prec, bool staged) {
+    return std::clamp((staged ? 24.0 : 23.0) - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
 }
 
-static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total, double few) {
+// staged: rows that come through LDS (Rader's): lines matter less, small blocks and
+// whole waves more.  120 cases of 11 to 2017 points, 2^20 to 2^23 in all: 4.8 % from the
+// best in the mean, by the terms of plain rows 10.4 % (441505 complex64 rows of 19
+// points 57 -> 42 us, 545587 of 13 47 -> 38).
+static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total, double few,
+                       bool staged) {
     const int es = prec ? 16 : 8, wps = prec ? 3 : 5, waves = m.threads / 64;
     const int by_waves = waves <= 8 ? wps * 4 / waves : wps / ((waves + 3) / 4);
     // blocks of exactly half a CU's LDS do not pair: complex128 columns of 640 points, 13107
@@ -613,10 +619,11 @@ static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, in
     // fewer blocks than CUs: smaller groups spread the work
     const double idle = blocks_total < 256 ? std::log2(256.0 / blocks_total) : 0.0;
     switch (lay) {
-    case MIX_ROWS:
-        return P + few * (serial / 64 + 0.1 * th) +
-               (1 - few) * (idle + 0.105 * work + 0.538 * inv + 0.113 * one + 0.056 * rl + 0.035 * rs + 0.029 * rl * rl +
-                            0.037 * rs * rs - 0.433 * th);
+    case MIX_ROWS: {
+        const double lines = 0.056 * rl + 0.035 * rs + 0.029 * rl * rl + 0.037 * rs * rs;
+        const double full = staged ? 0.8 * work + 0.3 * lines + 0.4 * th : 0.105 * work + lines - 0.433 * th;
+        return P + few * (serial / 64 + 0.1 * th) + (1 - few) * (idle + 0.538 * inv + 0.113 * one + full);
+    }
     case MIX_COLS:
         return P + few * (serial / 64 + 0.4 * th + 0.5 * idle + 0.023 * (seg128 + seg64)) +
                (1 - few) * (idle + 0.546 * work + 1.647 * inv + 3.575 * one + 1.155 * seg128 + 1.173 * seg64 - 1.645 * th);
@@ -655,8 +662,8 @@ int mix_passes(int64_t n) { return mix_min_passes(n, MIX_MAXPASS); }
 static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out,
                       double* cost = nullptr, int pad = 0) {
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
-    const double few = lay == MIX_TROWS ? 0.0 : mix_few(n, count, slices, prec);
-    const double conf = (1 - few) * (lay == MIX_ROWS ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012);
+    const double few = lay == MIX_TROWS ? 0.0 : mix_few(n, count, slices, prec, pad > 0);
+    const double conf = (1 - few) * (lay == MIX_ROWS ? (pad ? 0.05 : 0.005) : lay == MIX_COLS ? 0.203 : 0.012);
     const int minp = mix_min_passes(n, MIX_MAXPASS);
     if (minp > MIX_MAXPASS || (lay == MIX_TROWS ? n | 1 : n + pad) * es > 163840) return false;
     // Radices that the largest block holds, and the numbers of passes (bit p:
@@ -710,7 +717,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
                 m.lds = (int)lds;
                 m.threads = (m.g * m.tpt + 63) / 64 * 64;
                 m.rad = rad;
-                const double c = mix_cost(m, n, prec, lay, std::max<int64_t>(1, (count + m.g - 1) / m.g * slices), few);
+                const double c = mix_cost(m, n, prec, lay, std::max<int64_t>(1, (count + m.g - 1) / m.g * slices), few, pad > 0);
                 if (top.size() == KEEP && c >= top.back().first) continue;
                 auto it = top.begin();
                 while (it != top.end() && it->first <= c) ++it;
