@@ -322,15 +322,15 @@ static int emit_single(Plan& p, int di, const AxisJob& j, std::string& algo) {
     a.out_bd = out_bd;
     a.scale = j.scale;
     const int64_t gx = (count + k->tpb - 1) / k->tpb;
-    // Column groups that start and end on lines, or have none beside them, share
-    // nothing.  There XCD order pays from 64 MiB on; in what the caches hold it takes a block
+    // Column groups that start and end on lines share nothing.  There XCD order pays
+    // from 64 MiB on; from 8 MiB to there, in what the caches hold, it takes a block
     // away from the XCD whose L2 the pass before has filled (XCD -> plain order: complex128
-    // 8 x 32 x 4096 18.5 -> 13.3 us, 8 x 8 x 128 x 128 30.1 -> 24.4, complex64 64 x 16 x 1024 13.9 -> 11.2,
-    // 64 x 64 x 1024 28.1 -> 25.3; the four-step's columns want it at any size: 65536 x 16
-    // 13.2 against 15.9).
-    const bool apart = gx < 2 || (j.in_nd * es % 128 == 0 && j.out_nd * es % 128 == 0);
+    // 8 x 32 x 4096 18.5 -> 13.3 us, complex64 64 x 16 x 4096 31.2 -> 28.8, 64 x 64 x 1024 28.1 ->
+    // 25.3; the four-step's columns want it at any size: 65536 x 16 13.2 against 15.9).
+    const bool lines = j.in_nd * es % 128 == 0 && j.out_nd * es % 128 == 0;
+    const int64_t bytes = j.n * count * slices * es;
     a.xcd = var == VAR_COL && xcd_order(j.in_nd * es, j.out_nd * es) &&
-            (!apart || j.n * count * slices * es >= int64_t(64) << 20);
+            !(lines && bytes >= int64_t(8) << 20 && bytes < int64_t(64) << 20);
     Step s = make_step(k, a, gx, 1, var == VAR_ROW ? "row" : "col", gx * slices);
     // rows whose threads cover less than a line at a time: no streaming, which
     // would take the partial lines to memory one by one (complex64, 512 MiB: 8
@@ -533,7 +533,9 @@ struct MixShape {
     std::vector<int> rad;
     int tpt = 1, g = 1, threads = 64, lds = 0, pitch = 0;
 };
-enum MixLayout { MIX_ROWS = 0, MIX_COLS = 1, MIX_TROWS = 2 };   // VAR_ROW; VAR_COL and VAR_4A; VAR_4B
+// VAR_ROW and Rader's rows; VAR_COL and VAR_4A; VAR_4B; rows of the other kernels that
+// do more than one transform (real rows, padded Bluestein, convolution)
+enum MixLayout { MIX_ROWS = 0, MIX_COLS = 1, MIX_TROWS = 2, MIX_FUSED = 3 };
 
 // Mean number of LDS bank passes beyond the first of a wave's access to the
 // points addr(lane) (< 0: idle lane): the 64 banks of 4 bytes serve 256 bytes
@@ -582,23 +584,26 @@ static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout 
 // (columns) and 6.6 % (transposing rows) slower than the best one, 25 % at
 // worst.
 //
-// few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few; twice that for rows
-// through LDS, which compute longer on as much).  These are over
-// before their blocks have to share the CUs: a block's own time decides, the
-// passes and the points that a thread takes in turn, not the occupancy and the
-// conflicts.  On every shape of 360 row cases, 128 Rader rows and 184 column
-// cases of up to 2^20 points (10 to 8000 a transform, both precisions) the picks are 2.9, 2.7
-// and 3.5 % slower than the best in the mean, 21, 29 and 20 % at worst; by the
-// other terms alone 7.7, 6.2 and 28 %, 62, 33 and 125 % (complex64 columns 625 x 33 11.4 ->
-// 5.4 us, 1225 x 500 11.2 -> 8.3; 1245 rows of 421 points 11.2 -> 8.6).
-static double mix_few(int64_t n, int64_t count, int64_t slices, int prec, bool staged) {
-    return std::clamp((staged ? 24.0 : 23.0) - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
+// few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few); 16 and 32 for Rader's
+// rows, which compute longer on as much.  These are over before their blocks have to
+// share the CUs: a block's own time decides, the passes and the points that a
+// thread takes in turn, not the occupancy and (but for Rader's) the conflicts.
+// On every shape of 360 row and 184 column
+// cases of up to 2^20 points (10 to 8000 a transform, both precisions) the picks are 2.9
+// and 3.5 % slower than the best in the mean, 21 and 20 % at worst; by the
+// other terms alone 7.7 and 28 %, 62 and 125 % (complex64 columns 625 x 33 11.4 ->
+// 5.4 us, 1225 x 500 11.2 -> 8.3).  Columns in several slices and the fused kernels were
+// not among them and keep the other terms.
+static double mix_few(int64_t n, int64_t count, int64_t slices, int prec, MixLayout lay, bool staged) {
+    if (lay == MIX_TROWS || lay == MIX_FUSED || (lay == MIX_COLS && slices > 1)) return 0.0;
+    return std::clamp((staged ? 25.0 : 23.0) - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
 }
 
-// staged: rows that come through LDS (Rader's): lines matter less, small blocks and
-// whole waves more.  120 cases of 11 to 2017 points, 2^20 to 2^23 in all: 4.8 % from the
-// best in the mean, by the terms of plain rows 10.4 % (441505 complex64 rows of 19
-// points 57 -> 42 us, 545587 of 13 47 -> 38).
+// staged: rows that come through LDS (Rader's): lines matter less, small blocks,
+// whole waves and conflicts more.  386 cases of 11 to 2017 points, 2^14 to 2^23 in all: 2.7 %
+// from the best in the mean, 32 % at worst, by the terms of plain rows 6.0 and 42 %;
+// large complex128 launches keep those (4.4 to 7.8 % there, and some lengths 10 to 18 %
+// better: 38479 rows of 109 points 27.8 us against 32.9) (441505 complex64 rows of 19 points 57 -> 42 us, 545587 of 13 47 -> 38, 1245 of 421 11.2 -> 8.6).
 static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, int64_t blocks_total, double few,
                        bool staged) {
     const int es = prec ? 16 : 8, wps = prec ? 3 : 5, waves = m.threads / 64;
@@ -619,10 +624,12 @@ static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, in
     // fewer blocks than CUs: smaller groups spread the work
     const double idle = blocks_total < 256 ? std::log2(256.0 / blocks_total) : 0.0;
     switch (lay) {
-    case MIX_ROWS: {
+    case MIX_ROWS:
+    case MIX_FUSED: {
         const double lines = 0.056 * rl + 0.035 * rs + 0.029 * rl * rl + 0.037 * rs * rs;
-        const double full = staged ? 0.8 * work + 0.3 * lines + 0.4 * th : 0.105 * work + lines - 0.433 * th;
-        return P + few * (serial / 64 + 0.1 * th) + (1 - few) * (idle + 0.538 * inv + 0.113 * one + full);
+        const double full = staged && !prec ? 0.8 * work + inv + 0.113 * one + 0.3 * lines + 0.4 * th
+                                            : 0.105 * work + 0.538 * inv + 0.113 * one + lines - 0.433 * th;
+        return P + few * ((staged ? 1.5 : 1.0) * serial / 64 + 0.1 * th) + (1 - few) * (idle + full);
     }
     case MIX_COLS:
         return P + few * (serial / 64 + 0.4 * th + 0.5 * idle + 0.023 * (seg128 + seg64)) +
@@ -662,8 +669,10 @@ int mix_passes(int64_t n) { return mix_min_passes(n, MIX_MAXPASS); }
 static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t slices, MixShape& out,
                       double* cost = nullptr, int pad = 0) {
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
-    const double few = lay == MIX_TROWS ? 0.0 : mix_few(n, count, slices, prec, pad > 0);
-    const double conf = (1 - few) * (lay == MIX_ROWS ? (pad ? 0.05 : 0.005) : lay == MIX_COLS ? 0.203 : 0.012);
+    const bool rows = lay == MIX_ROWS || lay == MIX_FUSED;
+    const double few = mix_few(n, count, slices, prec, lay, pad > 0);
+    const double conf = pad ? 0.02 * few + (prec ? 0.005 : 0.1) * (1 - few)
+                            : (1 - few) * (rows ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012);
     const int minp = mix_min_passes(n, MIX_MAXPASS);
     if (minp > MIX_MAXPASS || (lay == MIX_TROWS ? n | 1 : n + pad) * es > 163840) return false;
     // Radices that the largest block holds, and the numbers of passes (bit p:
@@ -701,7 +710,7 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
             m.tpt = tpts[i];
             int last_g = 0;
             for (int w = 0; w < 6; ++w) {
-                if (lay == MIX_ROWS) {
+                if (rows) {
                     static constexpr int want[6] = {64, 128, 192, 256, 512, 0};
                     if (!want[w]) break;
                     m.g = (int)std::min<int64_t>(count, std::max(1, want[w] / m.tpt));
@@ -857,7 +866,7 @@ static int mix_args(Plan& p, int64_t n, MixLayout lay, int64_t count, int64_t sl
 
 int mix_row_launch(Plan& p, int64_t n, int64_t count, MixArgs& a, int* threads, int* lds) {
     MixShape m;
-    const int rc = mix_args(p, n, MIX_ROWS, count, 1, a, m);
+    const int rc = mix_args(p, n, MIX_FUSED, count, 1, a, m);
     a.k.count = count;
     *threads = m.threads;
     *lds = m.lds;
@@ -1370,7 +1379,7 @@ static int emit_mix_blue(Plan& p, int di, const AxisJob& j, int64_t m, bool rade
     MixBlueArgs a{};
     MixShape ms;
     int rc = blue_tables(p, j.n, m, 0.0, bt, rader ? BLUE_RADER : 0);
-    if (rc || (rc = mix_args(p, m, MIX_ROWS, j.count, j.slices, a.m, ms, rader ? 1 : 0))) return rc;
+    if (rc || (rc = mix_args(p, m, rader ? MIX_ROWS : MIX_FUSED, j.count, j.slices, a.m, ms, rader ? 1 : 0))) return rc;
     const void* fn = rader ? (prec ? mix_rader_kernel_c128() : mix_rader_kernel_c64())
                            : (prec ? mix_blue_kernel_c128() : mix_blue_kernel_c64());
     if ((rc = prep_dynamic_lds(fn, ms.lds))) return rc;
@@ -1446,7 +1455,7 @@ static int64_t blue_smooth_length(int64_t n, int64_t m, int prec, int64_t count,
     for (int64_t c = 2 * n - 1, seen = 0; c <= top && seen < 8; ++c) {
         MixShape ms;
         double cost;
-        if (smooth_schedule(c).empty() || !mix_shape(c, prec, MIX_ROWS, count, slices, ms, &cost)) continue;
+        if (smooth_schedule(c).empty() || !mix_shape(c, prec, MIX_FUSED, count, slices, ms, &cost)) continue;
         ++seen;
         // 256 complex64 points are two passes of the compile-time kernel: 2^23 points of
         // rows of 86 53.7 us, 89.6 padded to 175 = 7 x 5 x 5; of 79 54.3, 55.5 padded to
@@ -1915,7 +1924,7 @@ static int emit_real_rows(Plan& p, int di, int64_t n, int64_t rows, int64_t slic
     if (h >= 2 && (!is_pow2(h) || shortr) && !smooth_schedule(h).empty() && h <= gen_row_cap(prec)) {
         MixRealArgs a{};
         MixShape m;
-        if ((rc = mix_args(p, h, MIX_ROWS, rows, slices, a.m, m))) return rc;
+        if ((rc = mix_args(p, h, MIX_FUSED, rows, slices, a.m, m))) return rc;
         const void* fn = mix_real_kernel(prec, dir);
         if ((rc = prep_dynamic_lds(fn, m.lds))) return rc;
         a.wk = wk;
