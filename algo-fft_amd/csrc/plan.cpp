@@ -587,7 +587,7 @@ static double mix_bank_excess(const MixShape& m, int64_t n, int prec, MixLayout 
 // few: 1 for launches of up to 4 MiB, 0 from 8 MiB on (mix_few); 16 and 32 for Rader's
 // rows, which compute longer on as much.  These are over before their blocks have to
 // share the CUs: a block's own time decides, the passes and the points that a
-// thread takes in turn, not the occupancy and (but for Rader's) the conflicts.
+// thread takes in turn, little else (of columns not even the conflicts).
 // On every shape of 360 row and 184 column
 // cases of up to 2^20 points (10 to 8000 a transform, both precisions) the picks are 2.9
 // and 3.5 % slower than the best in the mean, 21 and 20 % at worst; by the
@@ -599,7 +599,7 @@ static double mix_few(int64_t n, int64_t count, int64_t slices, int prec, MixLay
     return std::clamp((staged ? 25.0 : 23.0) - std::log2((double)n * count * slices * (prec ? 16 : 8)), 0.0, 1.0);
 }
 
-// staged: rows that come through LDS (Rader's): lines matter less, small blocks,
+// staged: rows that come through LDS (Rader's): lines and the block size matter less,
 // whole waves and conflicts more.  386 cases of 11 to 2017 points, 2^14 to 2^23 in all: 2.7 %
 // from the best in the mean, 32 % at worst, by the terms of plain rows 6.0 and 42 %;
 // large complex128 launches keep those (4.4 to 7.8 % there, and some lengths 10 to 18 %
@@ -627,9 +627,9 @@ static double mix_cost(const MixShape& m, int64_t n, int prec, MixLayout lay, in
     case MIX_ROWS:
     case MIX_FUSED: {
         const double lines = 0.056 * rl + 0.035 * rs + 0.029 * rl * rl + 0.037 * rs * rs;
-        const double full = staged && !prec ? 0.8 * work + inv + 0.113 * one + 0.3 * lines + 0.4 * th
+        const double full = staged && !prec ? 0.2 * work + 0.538 * inv + 0.113 * one + 0.3 * lines - 0.2 * th
                                             : 0.105 * work + 0.538 * inv + 0.113 * one + lines - 0.433 * th;
-        return P + few * ((staged ? 1.5 : 1.0) * serial / 64 + 0.1 * th) + (1 - few) * (idle + full);
+        return P + few * (1.5 * serial / 64 + 0.1 * th) + (1 - few) * (idle + full);
     }
     case MIX_COLS:
         return P + few * (serial / 64 + 0.4 * th + 0.5 * idle + 0.023 * (seg128 + seg64)) +
@@ -671,8 +671,8 @@ static bool mix_shape(int64_t n, int prec, MixLayout lay, int64_t count, int64_t
     const int es = prec ? 16 : 8, maxth = prec ? MixCfg<double>::THREADS : MixCfg<float>::THREADS;
     const bool rows = lay == MIX_ROWS || lay == MIX_FUSED;
     const double few = mix_few(n, count, slices, prec, lay, pad > 0);
-    const double conf = pad ? 0.02 * few + (prec ? 0.005 : 0.1) * (1 - few)
-                            : (1 - few) * (rows ? 0.005 : lay == MIX_COLS ? 0.203 : 0.012);
+    const double conf = rows ? 0.02 * few + (pad && !prec ? 0.1 : 0.005) * (1 - few)
+                             : (1 - few) * (lay == MIX_COLS ? 0.203 : 0.012);
     const int minp = mix_min_passes(n, MIX_MAXPASS);
     if (minp > MIX_MAXPASS || (lay == MIX_TROWS ? n | 1 : n + pad) * es > 163840) return false;
     // Radices that the largest block holds, and the numbers of passes (bit p:
