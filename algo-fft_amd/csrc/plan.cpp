@@ -969,9 +969,9 @@ static int emit_gen_single(Plan& p, int di, const AxisJob& j, std::string& algo)
 // radices); ties go to the more balanced pair, then the smaller n1.  Fitted on 33
 // complex64 / complex128 lengths from 9000 to 10^6 on kernels with one radix of {2, 3,
 // 4, 5, 7, 8, 16} a pass: 5.4 % mean regret there, against 15.6 % for the power-of-two
-// part as the column factor.  On the composite radices it is 7.7 % over 599
-// shapes of the tuning records, 79 % at worst (12042240 as 735 x 16384 0.238 ms, 3136 x 3840
-// 0.133); wisdom and the cost model pick among the timed splits.  Lengths
+// part as the column factor.  On the composite radices it is 7.8 % over 599
+// shapes of the tuning records, 77 % at worst (12042240 as 735 x 16384 0.237 ms, 3136 x 3840
+// 0.134); wisdom and the cost model pick among the timed splits.  Lengths
 // with no such pair take the most balanced divisors within the caps.
 int64_t gen_fourstep_split(int64_t n, int prec) {
     const int64_t cap = gen_cap(prec), rcap = std::min<int64_t>(cap, 4096);
